@@ -419,8 +419,8 @@ mr_status mr_linear(const void* x, mr_dtype x_dtype, int32_t tokens, int64_t x_s
     if (w->in_features * (x_dtype == MR_F32 ? 4 : 2) < 16)
         return fail(MR_INVALID_SHAPE, "linear: an activation row of %lld %s values is under 16 bytes",
                     (long long)w->in_features, dtype_name(x_dtype));
-    if (tokens >= mr::PROJ_GEMM_MIN_TOKENS && x_dtype == MR_BF16 && w->dtype == MR_BF16) {
-        // many tokens: MFMA tiles
+    if (tokens > 1 && x_dtype == MR_BF16 && w->dtype == MR_BF16) {
+        // MFMA: a few tokens in tiles of 16, or many in tiles of 128 and 256
         mr::ProjGemmParams q{};
         q.x = (const uint16_t*)x;
         q.ldx = x_stride;
@@ -432,7 +432,12 @@ mr_status mr_linear(const void* x, mr_dtype x_dtype, int32_t tokens, int64_t x_s
         q.M = tokens;
         q.N = (int)w->out_features;
         q.K = (int)w->in_features;
-        if (mr::proj_gemm_ok(q)) {
+        const bool tiles = tokens >= mr::PROJ_GEMM_MIN_TOKENS && mr::proj_gemm_ok(q);
+        if (mr::skinny_gemm_ok(q) && (!tiles || mr::skinny_gemm_better(q.N, q.M, mrc::cu_count()))) {
+            const hipError_t e = mr::launch_skinny_gemm(q, mrc::cu_count(), (hipStream_t)stream);
+            return e == hipSuccess ? MR_OK : hip_fail(e, "linear launch");
+        }
+        if (tiles) {
             const hipError_t e = mr::launch_proj_gemm(q, mrc::cu_count(), (hipStream_t)stream);
             return e == hipSuccess ? MR_OK : hip_fail(e, "linear launch");
         }
@@ -1009,7 +1014,8 @@ mr_status proj_rows(const void* x, int32_t tokens, int64_t x_stride, const mr_pr
 mr_status proj_rows_stacked(const void* x, int32_t tokens, int64_t x_stride, const mr_projection* const* w,
                             void* const* y, const int64_t* y_stride, int n, void* stream) {
     mr::ProjGemmParams q[3];
-    bool stack = n > 1 && tokens >= mr::PROJ_GEMM_MIN_TOKENS;
+    bool stack = n > 1 && tokens >= mr::PROJ_GEMM_MIN_TOKENS, few = true;
+    int64_t rows = 0;
     for (int i = 0; stack && i < n; ++i) {
         q[i] = mr::ProjGemmParams{};
         q[i].x = (const uint16_t*)x;
@@ -1033,8 +1039,11 @@ mr_status proj_rows_stacked(const void* x, int32_t tokens, int64_t x_stride, con
             q[i].ldw = w[i]->dense.row_stride;
         }
         stack = stack && w[i]->kind == w[0]->kind && mr::proj_gemm_ok(q[i]);
+        few = few && mr::skinny_gemm_ok(q[i]);
+        rows += q[i].N;
     }
-    if (stack) {
+    // a call each where the few-token tiles are faster than the stack's
+    if (stack && !(few && mr::skinny_gemm_better(rows, tokens, mrc::cu_count()))) {
         const hipError_t e = mr::launch_proj_gemm_stack(q, n, mrc::cu_count(), (hipStream_t)stream);
         return e == hipSuccess ? MR_OK : hip_fail(e, "stacked projection launch");
     }

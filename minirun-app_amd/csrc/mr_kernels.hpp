@@ -204,11 +204,18 @@ struct ProjGemmStack {
     int32_t nseg;
     int32_t tile_end[3];
 };
-constexpr int PROJ_GEMM_MIN_TOKENS = 64;  // fewer tokens take the token-tile GEMV kernels
+constexpr int PROJ_GEMM_MIN_TOKENS = 64;  // fewer tokens take skinny.hip's tiles or the GEMV kernels
 bool proj_gemm_ok(const ProjGemmParams& p);  // shapes, alignment and formats the kernel takes
 hipError_t launch_proj_gemm(const ProjGemmParams& p, int cu_count, hipStream_t st);
 // n entries with one M, all dense or all affine, one output dtype; each proj_gemm_ok
 hipError_t launch_proj_gemm_stack(const ProjGemmParams* segs, int n, int cu_count, hipStream_t st);
+
+// ---------------------------------------------------------------- projections of a few tokens
+// The same product for a few tokens (skinny.hip), dense weights.
+bool skinny_gemm_ok(const ProjGemmParams& p);
+bool skinny_gemm_better(int64_t n, int m, int cus);  // than launch_proj_gemm
+hipError_t launch_skinny_gemm(const ProjGemmParams& p, int cu_count, hipStream_t st);
+
 hipError_t launch_prefill_attn(const PrefillAttnParams& p, hipStream_t st);
 
 // ---------------------------------------------------------------- top-k
