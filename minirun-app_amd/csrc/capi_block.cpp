@@ -377,8 +377,8 @@ mr_status mr_affine_matmul(const void* x, mr_dtype x_dtype, int32_t tokens, int6
     g.y_stride_row = 1;
     g.y_stride_token = y_stride;
     g.force_generic = !aligned16(w->packed);  // the fused kernel loads 16-byte row chunks
-    if (tokens >= mr::PROJ_GEMM_MIN_TOKENS && x_dtype == MR_BF16) {
-        // many tokens: dequantized k-tiles into LDS and MFMA
+    if (tokens > 1 && x_dtype == MR_BF16) {
+        // MFMA: a few tokens in tiles of 16, or many in tiles of 128 and 256
         mr::ProjGemmParams q{};
         q.x = (const uint16_t*)x;
         q.ldx = x_stride;
@@ -394,7 +394,12 @@ mr_status mr_affine_matmul(const void* x, mr_dtype x_dtype, int32_t tokens, int6
         q.M = tokens;
         q.N = (int)w->out_features;
         q.K = (int)w->in_features;
-        if (mr::proj_gemm_ok(q)) {
+        const bool tiles = tokens >= mr::PROJ_GEMM_MIN_TOKENS && mr::proj_gemm_ok(q);
+        if (mr::skinny_gemm_ok(q) && (!tiles || mr::skinny_gemm_better(q.N, q.M, true, mrc::cu_count()))) {
+            const hipError_t e = mr::launch_skinny_gemm(q, mrc::cu_count(), (hipStream_t)stream);
+            return e == hipSuccess ? MR_OK : hip_fail(e, "affine matmul launch");
+        }
+        if (tiles) {
             const hipError_t e = mr::launch_proj_gemm(q, mrc::cu_count(), (hipStream_t)stream);
             return e == hipSuccess ? MR_OK : hip_fail(e, "affine matmul launch");
         }
@@ -420,7 +425,7 @@ mr_status mr_linear(const void* x, mr_dtype x_dtype, int32_t tokens, int64_t x_s
         return fail(MR_INVALID_SHAPE, "linear: an activation row of %lld %s values is under 16 bytes",
                     (long long)w->in_features, dtype_name(x_dtype));
     if (tokens > 1 && x_dtype == MR_BF16 && w->dtype == MR_BF16) {
-        // MFMA: a few tokens in tiles of 16, or many in tiles of 128 and 256
+        // MFMA, as in mr_affine_matmul
         mr::ProjGemmParams q{};
         q.x = (const uint16_t*)x;
         q.ldx = x_stride;
@@ -433,7 +438,7 @@ mr_status mr_linear(const void* x, mr_dtype x_dtype, int32_t tokens, int64_t x_s
         q.N = (int)w->out_features;
         q.K = (int)w->in_features;
         const bool tiles = tokens >= mr::PROJ_GEMM_MIN_TOKENS && mr::proj_gemm_ok(q);
-        if (mr::skinny_gemm_ok(q) && (!tiles || mr::skinny_gemm_better(q.N, q.M, mrc::cu_count()))) {
+        if (mr::skinny_gemm_ok(q) && (!tiles || mr::skinny_gemm_better(q.N, q.M, false, mrc::cu_count()))) {
             const hipError_t e = mr::launch_skinny_gemm(q, mrc::cu_count(), (hipStream_t)stream);
             return e == hipSuccess ? MR_OK : hip_fail(e, "linear launch");
         }
@@ -1043,7 +1048,7 @@ mr_status proj_rows_stacked(const void* x, int32_t tokens, int64_t x_stride, con
         rows += q[i].N;
     }
     // a call each where the few-token tiles are faster than the stack's
-    if (stack && !(few && mr::skinny_gemm_better(rows, tokens, mrc::cu_count()))) {
+    if (stack && !(few && mr::skinny_gemm_better(rows, tokens, w[0]->kind == MR_PROJ_AFFINE, mrc::cu_count()))) {
         const hipError_t e = mr::launch_proj_gemm_stack(q, n, mrc::cu_count(), (hipStream_t)stream);
         return e == hipSuccess ? MR_OK : hip_fail(e, "stacked projection launch");
     }

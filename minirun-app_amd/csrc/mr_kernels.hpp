@@ -211,10 +211,21 @@ hipError_t launch_proj_gemm(const ProjGemmParams& p, int cu_count, hipStream_t s
 hipError_t launch_proj_gemm_stack(const ProjGemmParams* segs, int n, int cu_count, hipStream_t st);
 
 // ---------------------------------------------------------------- projections of a few tokens
-// The same product for a few tokens (skinny.hip), dense weights.
+// The same product for a few tokens (skinny.hip); affine weights in groups
+// that are a multiple of 64.
 bool skinny_gemm_ok(const ProjGemmParams& p);
-bool skinny_gemm_better(int64_t n, int m, int cus);  // than launch_proj_gemm
+bool skinny_gemm_better(int64_t n, int m, bool affine, int cus);  // than launch_proj_gemm
 hipError_t launch_skinny_gemm(const ProjGemmParams& p, int cu_count, hipStream_t st);
+// Routed: pair i (token i / per_token) reads expert ids[i]'s N weight rows of
+// the stacked affine weight and writes y row i; zeros for an id out of range.
+// M counts the x rows.
+struct SkinnyRoute {
+    const int32_t* ids;
+    int32_t pairs, per_token, experts;
+};
+bool skinny_routed_ok(const ProjGemmParams& p, const SkinnyRoute& route);
+bool skinny_routed_better(int64_t pairs, int64_t experts);  // than a GEMV per pair
+hipError_t launch_skinny_routed(const ProjGemmParams& p, const SkinnyRoute& route, hipStream_t st);
 
 hipError_t launch_prefill_attn(const PrefillAttnParams& p, hipStream_t st);
 

@@ -1,12 +1,14 @@
 // Projections of a few tokens on MFMA: y[T][N] = x[T][K] . W[N][K]^T for the
 // calls between one token (the GEMV kernels) and a prompt (gemm.hip): a batch
-// of decodes, speculative tokens, short prompts.  k3Linear (Linear.swift:55-57).
+// of decodes, speculative tokens, short prompts, and the tokens that a router
+// sends to one expert.  k3Linear (Linear.swift:55-57), affineMM
+// (AffineWeights.swift:239-254), affineGatherMM (AffineWeights.swift:255-318).
 //
 // What bounds it: the weights' bytes from HBM while T is small (each weight is
 // read once per 16 TT tokens), the activations' bytes from L2 after that
 // (every workgroup reads all of its tokens' rows).  A workgroup of 8 waves
 // owns 16 RT weight rows and 16 TT tokens, and its waves split K: wave w takes
-// ring entries w, w + 8, ... of 32 k.  Each wave
+// ring entries w, w + 8, ... of 32 k (dense) or 128 k (4-bit).  Each wave
 // streams its own entries into its own LDS ring of S entries by DMA and waits
 // for its own vmcnt, so the loop has no barrier; an entry's fragments are read
 // to registers, the slot is refilled at once, then the products run.  The
@@ -23,6 +25,17 @@
 // Short chains of MFMAs start from zero and are added to the running sums by
 // fp32 adds: fewer roundings at the size of the whole sum (with one chain per
 // wave the error against 64 bits is a third larger).
+//
+// Affine weights are not dequantized: a lane's weight row has one scale and
+// one bias per group, so
+//   y_o += s_og * (sum_{i in g} x_i q_oi) + b_og * (sum_{i in g} x_i)
+// with both inner sums on MFMA (q = 0..15 is exact in bf16; the sum of x is a
+// product with ones) and the two multiply-adds in fp32.  A nibble becomes bf16
+// by v_cvt_scalef32_pk_bf16_fp8: the e4m3 codes 0..15 are q * 2^-9 (0..7
+// subnormal), and the scale 2^9 makes them q.  An output that is not finite
+// that way (an infinite activation, or a sum that overflows without its
+// scale) is computed again from dequantized weights, one by one, so it holds
+// what those give.
 #include <algorithm>
 
 #include "mr_kernels.hpp"
@@ -182,6 +195,272 @@ __global__ void __launch_bounds__(64 * NW) skinny_dense_kernel(ProjGemmParams p,
     });
 }
 
+// ---------------------------------------------------------------- 4-bit affine
+// eight nibbles of a word as bf16 0..15, in their order
+__device__ __forceinline__ bf16x8 nibbles_bf16(uint32_t w) {
+    const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;  // nibbles 0,2,4,6 / 1,3,5,7
+    const uint32_t a = __builtin_amdgcn_perm(hi, lo, 0x05010400u), b = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
+    const u32x4 v = {__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(a, 512.f, false)),
+                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(a, 512.f, true)),
+                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 512.f, false)),
+                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 512.f, true))};
+    return __builtin_bit_cast(bf16x8, v);
+}
+
+template <int SDT>
+__device__ __forceinline__ float sk_scale(uint32_t v) {
+    return SDT == 0 ? __uint_as_float(v << 16) : (SDT == 1 ? f16_bits_to_f32((uint16_t)v) : __uint_as_float(v));
+}
+
+// one output from dequantized weights, in order
+template <int SDT>
+__device__ __forceinline__ float sk_affine_dot(const uint16_t* x, const uint32_t* packed, const void* scales,
+                                               const void* biases, int K, int group) {
+    float acc = 0.f;
+#pragma unroll 1
+    for (int i = 0; i < K; ++i) {
+        const int g = i / group;
+        const float s = sk_scale<SDT>(SDT == 2 ? ((const uint32_t*)scales)[g] : ((const uint16_t*)scales)[g]);
+        const float b = sk_scale<SDT>(SDT == 2 ? ((const uint32_t*)biases)[g] : ((const uint16_t*)biases)[g]);
+        const float qv = (float)((packed[i >> 3] >> (4 * (i & 7))) & 15u);
+        acc = fmaf(bf16_bits_to_f32(x[i]), add_rn(mul_rn(s, qv), b), acc);
+    }
+    return acc;
+}
+
+__device__ __forceinline__ void dma4_buf(i32x4 rsrc, uint32_t voff, const void* lds_dst_wave_base) {
+    const uint32_t m0 = (uint32_t)(uintptr_t)lds_dst_wave_base;
+    asm volatile("buffer_load_dword %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "{m0}"(m0) : "memory");
+}
+
+constexpr int SK_SCAN = 4096;  // routed: pairs per scan
+
+// Ring entry: two groups (128 k); W [16 RT rows][64 B] (chunk c of row r in
+// slot c ^ ((r >> 2) & 3)), x [16 TT rows][256 B] (slot c ^ (r % 16)), then per
+// (row, group) the dword that holds its scale and the one that holds its bias.
+//
+// Measured as above, before (one wave per output, or the 128-row tiles of
+// gemm.hip) -> now: 7168 x 16384, 13 tokens 2280 -> 22 us, 24 tokens 4150 -> 27
+// us, 64 tokens 661 -> 44 us; 24576 x 1536, 13 tokens 780 -> 11 us.  One ring
+// entry per wave (S = 1, all 8 waves' entries in flight) is as fast as three.
+//
+// Routed: workgroup (expert, row tile).  It scans the ids for its expert's
+// (token, slot) pairs, up to SK_SCAN pairs at a time, and takes them 16 TT at
+// a time; expert index `experts` stands for the ids out of range, whose
+// outputs are zeros.  768 x 2048, 128 experts, 8 per token: 200 tokens 223 ->
+// 50 us, 64 tokens 67 -> 39 us; 4 waves and 16 tokens per workgroup, so
+// that four of them share a CU: a workgroup is a chain of waits (ids, rows,
+// sums), and 8 waves or 32 tokens each were slower.
+template <int RT, int TT, int S, int SDT, bool ROUTED, int NW>
+__global__ void __launch_bounds__(64 * NW) skinny_affine_kernel(ProjGemmParams p, SkinnyRoute route, int blocks) {
+    static_assert(RT <= 2, "one DMA of scales per entry");
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    constexpr int NI = RT + 4 * TT + 2, XOFF = 1024 * RT, SOFF = XOFF + 4096 * TT, ENTRY = SOFF + 512;
+    static_assert((S - 1) * NI < 64, "vmcnt range");
+    const int tid = threadIdx.x, l = tid & 63, q = l >> 4, lr = l & 15;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int tile, tb = 0, e = 0;
+    const int n_tiles = (p.N + 16 * RT - 1) / (16 * RT);
+    if (ROUTED) {
+        e = blockIdx.x / n_tiles;
+        tile = blockIdx.x - e * n_tiles;
+    } else {
+        sk_tile(blockIdx.x, blocks, tile, tb);
+        if (tile >= n_tiles) return;
+    }
+    const int n0 = tile * 16 * RT, rows = min(16 * RT, p.N - n0);
+    const int G = p.K / 64, nblk = (G + 1) / 2;
+    const uint32_t wrow = (uint32_t)p.K / 2, srow = (uint32_t)(p.K / p.group) * (SDT == 2 ? 4 : 2);
+    const int gpl = p.group / 64;  // 64-groups per scale
+    const int n = w < nblk ? (nblk - 1 - w) / NW + 1 : 0;  // this wave's entries
+    const int64_t wr0 = (int64_t)(ROUTED ? min(e, route.experts - 1) : 0) * p.N + n0;
+    const char* wbase = (const char*)p.packed + wr0 * wrow;
+    const char *sbase = (const char*)p.scales + wr0 * srow, *bbase = (const char*)p.biases + wr0 * srow;
+    const i32x4 wres = uniform_rsrc(wbase, (uint32_t)rows * wrow);
+    // (2-byte scales: through the dword that holds the last one)
+    const i32x4 sres = uniform_rsrc(sbase, ((uint32_t)rows * srow + 3u) & ~3u);
+    const i32x4 bres = uniform_rsrc(bbase, ((uint32_t)rows * srow + 3u) & ~3u);
+    uint32_t wo[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+        const int row = 16 * r + (l >> 2);
+        wo[r] = row < rows ? (uint32_t)row * wrow + 16u * ((l & 3) ^ ((l >> 4) & 3)) : SK_OOB_ROW;
+    }
+    // lane l of the scale DMA: row l / 2, group l % 2 of the entry
+    const uint32_t so = (l >> 1) < rows ? (uint32_t)(l >> 1) * srow : SK_OOB_ROW;
+    char* ring = lds + w * S * ENTRY;
+    auto issue_w = [&](int i, char* ent) {
+        const int blk = w + NW * i;
+        const uint32_t o = i < n ? 64u * blk : SK_OOB_K;
+#pragma unroll
+        for (int r = 0; r < RT; ++r) dma16_buf(wres, wo[r] + o, ent + 1024 * r);
+        const int g = min(2 * blk + (l & 1), G - 1);  // a group past the last is not used
+        const uint32_t gs = (uint32_t)(gpl == 1 ? g : g / gpl) * (SDT == 2 ? 4 : 2);
+        const uint32_t sv = i < n ? (so + gs) & ~3u : SK_OOB_K;
+        dma4_buf(sres, sv, ent + SOFF);
+        dma4_buf(bres, sv, ent + SOFF + 256);
+    };
+    const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
+    f32x4 tot[RT][TT];
+    // the products of `toks` tokens: x row and y row of token i from row_of
+    auto tokens = [&](int toks, const uint16_t* xb, int64_t xbytes, auto xrow_of, auto yrow_of) {
+        const i32x4 xres = uniform_rsrc(xb, (uint32_t)xbytes);
+        // lane l of DMA u: row 4 u + l / 16, slot l % 16, chunk slot ^ (row % 16)
+        uint32_t xo[TT][4];
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int rt = 4 * u + q, tok = 16 * t + rt;
+                xo[t][u] = tok < toks ? (uint32_t)(xrow_of(tok) * p.ldx * 2) + 16u * (lr ^ rt) : SK_OOB_ROW;
+            }
+        auto issue = [&](int i, int slot) {
+            char* ent = ring + slot * ENTRY;
+            issue_w(i, ent);
+            const uint32_t o = i < n ? 256u * (uint32_t)(w + NW * i) : SK_OOB_K;
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) dma16_buf(xres, xo[t][u] + o, ent + XOFF + 4096 * t + 1024 * u);
+        };
+        f32x4 part[RT][TT];
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int t = 0; t < TT; ++t) tot[r][t] = part[r][t] = f32x4{};
+#pragma unroll
+        for (int s = 0; s < S; ++s) issue(s, s);
+        int slot = 0;
+        for (int i = 0; i < n; ++i) {
+            wait_vmcnt<(S - 1) * NI>();
+            const char* ent = ring + slot * ENTRY;
+            const int blk = w + NW * i;
+            u32x2 fw[RT][2], sv[RT], bv[RT];
+            bf16x8 fx[TT][2][2];
+#pragma unroll
+            for (int r = 0; r < RT; ++r) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    fw[r][j] = *(const u32x2*)(ent + 1024 * r + 64 * lr + 16 * ((2 * j + (q >> 1)) ^ (lr >> 2)) + 8 * (q & 1));
+                sv[r] = *(const u32x2*)(ent + SOFF + 128 * r + 8 * lr);
+                bv[r] = *(const u32x2*)(ent + SOFF + 256 + 128 * r + 8 * lr);
+            }
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int s = 0; s < 2; ++s)
+                        fx[t][j][s] = *(const bf16x8*)(ent + XOFF + 4096 * t + 256 * lr + 16 * ((8 * j + 2 * q + s) ^ lr));
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0xc07f);  // the same, known to the compiler
+            __builtin_amdgcn_sched_barrier(0);
+            issue(i + S, slot);
+            slot = slot + 1 == S ? 0 : slot + 1;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int g = 2 * blk + j;
+                const bool live = g < G;
+                f32x4 xs[TT];
+#pragma unroll
+                for (int t = 0; t < TT; ++t) xs[t] = mfma16(fx[t][j][1], ones, mfma16(fx[t][j][0], ones, f32x4{}));
+#pragma unroll
+                for (int r = 0; r < RT; ++r) {
+                    uint32_t sw = sv[r][j], bw = bv[r][j];
+                    if (SDT != 2) {  // the half that holds it
+                        const uint32_t sh =
+                            (((16 * r + lr) * (srow >> 1) + (uint32_t)(gpl == 1 ? g : g / gpl)) & 1u) * 16u;
+                        sw = (sw >> sh) & 0xffffu;
+                        bw = (bw >> sh) & 0xffffu;
+                    }
+                    const float s = live ? sk_scale<SDT>(sw) : 0.f, b = live ? sk_scale<SDT>(bw) : 0.f;
+                    const bf16x8 w0 = nibbles_bf16(fw[r][j][0]), w1 = nibbles_bf16(fw[r][j][1]);
+#pragma unroll
+                    for (int t = 0; t < TT; ++t) {
+                        const f32x4 d = mfma16(fx[t][j][1], w1, mfma16(fx[t][j][0], w0, f32x4{}));
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) part[r][t][k] = fmaf(b, xs[t][k], fmaf(s, d[k], part[r][t][k]));
+                    }
+                }
+            }
+            if ((i & 3) == 3 || i + 1 == n) {
+#pragma unroll
+                for (int r = 0; r < RT; ++r)
+#pragma unroll
+                    for (int t = 0; t < TT; ++t) {
+                        tot[r][t] += part[r][t];
+                        part[r][t] = f32x4{};
+                    }
+            }
+        }
+        wait_vmcnt<0>();
+        sk_reduce<RT, TT, NW>(lds, tot, [&](int r, int t, int lane, f32x4 v) {
+            const int nn = 16 * r + (lane & 15);
+            if (nn >= rows) return;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int m = 16 * t + 4 * (lane >> 4) + i;
+                if (m >= toks) break;
+                float y = v[i];
+                if (!(fabsf(y) < INFINITY))
+                    y = sk_affine_dot<SDT>(xb + xrow_of(m) * p.ldx, (const uint32_t*)(wbase + (int64_t)nn * wrow),
+                                           sbase + (int64_t)nn * srow, bbase + (int64_t)nn * srow, p.K, p.group);
+                const int64_t o = yrow_of(m) * p.ldy + n0 + nn;
+                if (p.y_f32)
+                    ((float*)p.y)[o] = y;
+                else
+                    ((uint16_t*)p.y)[o] = f32_to_bf16_bits(y);
+            }
+        });
+    };
+    if constexpr (!ROUTED) {
+        const int m0 = tb * 16 * TT, toks = min(16 * TT, p.M - m0);
+        tokens(toks, p.x + (int64_t)m0 * p.ldx, ((int64_t)(toks - 1) * p.ldx + p.K) * 2,
+               [](int i) { return (int64_t)i; }, [&](int i) { return (int64_t)(m0 + i); });
+    } else {
+        constexpr int IDS = SK_SCAN / (64 * NW);  // ids per thread
+        uint16_t* list = (uint16_t*)(lds + std::max(NW * S * ENTRY, NW * RT * TT * 1024));
+        int& count = *(int*)(list + SK_SCAN);
+        for (int base = 0; base < route.pairs; base += SK_SCAN) {
+            int id[IDS];
+#pragma unroll
+            for (int u = 0; u < IDS; ++u) id[u] = route.ids[min(base + u * (64 * NW) + tid, route.pairs - 1)];
+            if (tid == 0) count = 0;
+            __syncthreads();
+            // in no particular order: a token's products do not depend on
+            // its place among the others
+#pragma unroll
+            for (int u = 0; u < IDS; ++u) {
+                const int i = u * (64 * NW) + tid;
+                const bool bad = (uint32_t)id[u] >= (uint32_t)route.experts;
+                if (base + i < route.pairs && (e == route.experts ? bad : id[u] == e))
+                    list[atomicAdd(&count, 1)] = (uint16_t)i;
+            }
+            __syncthreads();
+            const int cnt = count;
+            for (int i0 = 0; i0 < cnt; i0 += 16 * TT) {
+                const int toks = min(16 * TT, cnt - i0);
+                if (e == route.experts) {
+                    for (int i = tid; i < toks * rows; i += 64 * NW) {
+                        const int64_t o = (int64_t)(base + list[i0 + i / rows]) * p.ldy + n0 + i % rows;
+                        if (p.y_f32)
+                            ((float*)p.y)[o] = 0.f;
+                        else
+                            ((uint16_t*)p.y)[o] = 0;
+                    }
+                } else {
+                    auto pair = [&](int i) { return base + (int)list[i0 + i]; };
+                    tokens(toks, p.x, ((int64_t)(p.M - 1) * p.ldx + p.K) * 2,
+                           [&](int i) { return (int64_t)((uint32_t)pair(i) / (uint32_t)route.per_token); },
+                           [&](int i) { return (int64_t)pair(i); });
+                    __syncthreads();  // the partial sums are read before the ring is written again
+                }
+            }
+            __syncthreads();  // the list and count too
+        }
+    }
+}
+
 template <typename K>
 hipError_t set_lds(K kern, size_t lds) {
     return lds > 65536 ? hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)
@@ -200,13 +479,49 @@ hipError_t launch_dense(const ProjGemmParams& p, hipStream_t st) {
     return hipGetLastError();
 }
 
+template <int RT, int TT, int S, int SDT, bool ROUTED, int NW>
+hipError_t launch_affine(const ProjGemmParams& p, const SkinnyRoute& route, hipStream_t st) {
+    constexpr size_t ring = std::max<size_t>((size_t)NW * S * (1024 * RT + 4096 * TT + 512), (size_t)NW * RT * TT * 1024);
+    constexpr size_t lds = ring + (ROUTED ? SK_SCAN * 2 + 4 : 0);
+    static_assert(lds <= 163840, "LDS");
+    const auto kern = skinny_affine_kernel<RT, TT, S, SDT, ROUTED, NW>;
+    const hipError_t e = set_lds(kern, lds);
+    if (e != hipSuccess) return e;
+    const int tiles = (p.N + 16 * RT - 1) / (16 * RT), blocks = (p.M + 16 * TT - 1) / (16 * TT);
+    const unsigned grid = ROUTED ? (unsigned)(tiles * (route.experts + 1)) : (unsigned)((tiles + 7) / 8 * 8 * blocks);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * NW), lds, st, p, route, blocks);
+    return hipGetLastError();
+}
+
+template <int RT, int TT, int S, bool ROUTED, int NW>
+hipError_t launch_affine_sdt(const ProjGemmParams& p, const SkinnyRoute& route, hipStream_t st) {
+    if (p.scale_dtype == 0) return launch_affine<RT, TT, S, 0, ROUTED, NW>(p, route, st);
+    if (p.scale_dtype == 1) return launch_affine<RT, TT, S, 1, ROUTED, NW>(p, route, st);
+    return launch_affine<RT, TT, S, 2, ROUTED, NW>(p, route, st);
+}
+
+bool affine_rows_ok(const ProjGemmParams& p) {
+    if (p.bits != 4 || p.group % 64 || p.K % p.group || ((uintptr_t)p.packed & 15)) return false;
+    if (((uintptr_t)p.scales | (uintptr_t)p.biases) & 3) return false;
+    // 2-byte scales are read by the dword that holds them: every tile's first
+    // one and the end of all rows on a dword
+    if (p.scale_dtype != 2 && ((int64_t)p.N * (p.K / p.group)) % 2) return false;
+    return (int64_t)64 * (p.K / 2) < (1 << 30);
+}
+
 }  // namespace
 
 bool skinny_gemm_ok(const ProjGemmParams& p) {
     if (p.M <= 0 || p.N <= 0 || p.K < 32 || p.K % 32 || ((uintptr_t)p.x & 15) || p.ldx % 8 || p.ldx < p.K) return false;
     if ((int64_t)64 * p.ldx * 2 >= (1 << 30)) return false;  // byte offsets of one token block's rows
     if (((int64_t)p.N / 16 + 8) * ((int64_t)p.M / 16 + 1) > INT32_MAX) return false;  // workgroups
-    return !p.packed && p.w && ((uintptr_t)p.w & 15) == 0 && p.ldw % 8 == 0 && p.ldw >= p.K && (int64_t)64 * p.ldw * 2 < (1 << 30);
+    if (p.packed) return affine_rows_ok(p);
+    return p.w && ((uintptr_t)p.w & 15) == 0 && p.ldw % 8 == 0 && p.ldw >= p.K && (int64_t)64 * p.ldw * 2 < (1 << 30);
+}
+
+bool skinny_routed_ok(const ProjGemmParams& p, const SkinnyRoute& route) {
+    return p.packed && skinny_gemm_ok(p) && (int64_t)p.M * p.ldx * 2 < (1 << 30) && route.pairs <= INT32_MAX - SK_SCAN &&
+           ((int64_t)p.N / 32 + 1) * (route.experts + 1) < INT32_MAX;
 }
 
 namespace {
@@ -237,19 +552,40 @@ int dense_rt(int64_t n, int m, int cus) {
 
 // Against gemm.hip's tiles, both in rounds of one workgroup per CU.  Dense: a
 // unit of dense_cost takes 1.65 ns per k (52 us at 12288 x 7168, 64 tokens),
-// a round of 128-row tiles 17.5 ns per k (128 us there).
-bool skinny_gemm_better(int64_t n, int m, int cus) {
+// a round of 128-row tiles 17.5 ns per k (128 us there).  Affine: a round of
+// 32 rows x 64 tokens takes 2.7 ns per k (44 us at K = 16384), a round of
+// 128-row tiles 40 ns (661 us).
+bool skinny_gemm_better(int64_t n, int m, bool affine, int cus) {
     if (m < PROJ_GEMM_MIN_TOKENS) return true;
     const int64_t tiles = (int64_t)((m + 127) / 128) * ((n + 255) / 256), rounds = (tiles + cus - 1) / cus;
+    if (affine) {
+        const int64_t wgs = (int64_t)((n + 31) / 32) * ((m + 63) / 64);
+        return (double)((wgs + cus - 1) / cus) * 2.7 < 40. * rounds;
+    }
     return dense_cost(n, m, dense_rt(n, m, cus), cus) * 1.65 < 17.5 * rounds;
 }
 
 hipError_t launch_skinny_gemm(const ProjGemmParams& p, int cu_count, hipStream_t st) {
     const int tt = token_tiles(p.M);
+    if (p.packed) {
+        const SkinnyRoute none{};
+        if (tt == 1) return launch_affine_sdt<2, 1, 1, false, 8>(p, none, st);
+        if (tt == 2) return launch_affine_sdt<2, 2, 1, false, 8>(p, none, st);
+        return launch_affine_sdt<2, 4, 1, false, 8>(p, none, st);
+    }
     const int rt = dense_rt(p.N, p.M, cu_count);
     if (tt == 1) return rt == 1 ? launch_dense<1, 1, 4, 8>(p, st) : (rt == 2 ? launch_dense<2, 1, 3, 8>(p, st) : launch_dense<3, 1, 2, 8>(p, st));
     if (tt == 2) return rt == 1 ? launch_dense<1, 2, 3, 8>(p, st) : (rt == 2 ? launch_dense<2, 2, 2, 8>(p, st) : launch_dense<3, 2, 2, 8>(p, st));
     return rt == 1 ? launch_dense<1, 4, 2, 8>(p, st) : (rt == 2 ? launch_dense<2, 4, 3, 8>(p, st) : launch_dense<3, 4, 2, 8>(p, st));
+}
+
+// A workgroup per expert and row tile pays once an expert has a few tokens; a
+// GEMV per (token, slot) is faster below (128 experts: 128 pairs 20 against 26
+// us, 512 pairs 67 against 39 us)
+bool skinny_routed_better(int64_t pairs, int64_t experts) { return pairs >= 2 * experts; }
+
+hipError_t launch_skinny_routed(const ProjGemmParams& p, const SkinnyRoute& route, hipStream_t st) {
+    return launch_affine_sdt<2, 1, 1, true, 4>(p, route, st);
 }
 
 }  // namespace mr

@@ -1,10 +1,12 @@
-"""Projections of a few tokens (mr_linear, 2 to about 100 tokens) on MFMA, at the
-edges of their tiles: 16 tokens, 16 to 48 weight rows, 32 k per wave and ring
-entry, 8 waves over K.
+"""Projections of a few tokens (mr_linear, mr_affine_matmul, 2 to about 100
+tokens) and routed experts (mr_affine_gather_matmul) on MFMA, at the edges of
+their tiles: 16 tokens, 16 to 48 weight rows, 32 (dense) or 128 (4-bit) k per
+wave and ring entry, 8 waves over K.
 
 Reference: float64 numpy over the exact float32 weights.  Bar, elementwise: a
 sum over K in fp32 with at most K roundings of partial sums no larger than
-sum |x| |w|, times 2^-24 each; the chains are shorter than K / 8, so K / 8 + 32 of them are
+sum |x| |w| (affine: of the scaled and the bias part, sum |x| (|s| q + |b|)),
+times 2^-24 each; the chains are shorter than K / 8, so K / 8 + 32 of them are
 allowed; bf16 outputs add half a unit in the last place (2^-9 relative, and
 again for the sum's own error on a tie)."""
 import numpy as np
@@ -12,6 +14,7 @@ import pytest
 
 import oracle as O
 from test_gpu_block import dev, f32, sync
+from test_gpu_proj_gemm import affine_operand
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +58,55 @@ def test_linear_few_tokens(M, tokens, out_f, in_f, x_pad, ydt):
     sync()
     xd, wd = O.bf16_to_f32(x[:, :in_f]).astype(np.float64), O.bf16_to_f32(w).astype(np.float64)
     compare(y, xd @ wd.T, np.abs(xd) @ np.abs(wd).T, in_f, ydt)
+
+
+def dequant(packed, sa, ba, code, group):
+    """(exact float32 weights, |s| q + |b|) as float64"""
+    conv = {O.BF16: O.bf16_to_f32, O.F16: lambda a: a.view(np.float16).astype(np.float32), O.F32: lambda a: a}[code]
+    q = ((packed[..., None] >> np.arange(0, 32, 4, dtype=np.uint32)) & 15).reshape(*packed.shape[:-1], -1)
+    s, b = np.repeat(conv(sa), group, -1), np.repeat(conv(ba), group, -1)
+    w = (s * q.astype(np.float32)).astype(np.float32) + b
+    return w.astype(np.float64), (np.abs(s) * q + np.abs(b)).astype(np.float64)
+
+
+@pytest.mark.parametrize("tokens", [2, 16, 17, 33, 64, 65])
+@pytest.mark.parametrize("out_f,in_f,group,sdt,x_pad,ydt", [
+    (6, 64, 64, "bf16", 0, "f32"),       # one group: half a ring entry
+    (40, 192, 64, "f16", 8, "f32"),      # an odd group count; ragged row tile
+    (33, 1152, 128, "f32", 0, "bf16"),   # 9 entries, one scale per entry
+    (34, 1088, 64, "bf16", 0, "bf16"),   # 17 groups: scales on both halves of a dword
+    (64, 2048, 256, "bf16", 16, "f32"),
+])
+def test_affine_few_tokens(M, tokens, out_f, in_f, group, sdt, x_pad, ydt):
+    print(f"affine few T={tokens} [{out_f}, {in_f}] g={group} scales={sdt} pad={x_pad} y={ydt}", flush=True)
+    packed, sa, ba, code, ts, tb = affine_operand(f"af.{out_f}.{in_f}", out_f, in_f, group, sdt)
+    x = O.normal_bf16(f"af.x.{tokens}.{in_f}", (tokens, in_f + x_pad))
+    w = M.AffineWeights(dev(packed), ts, tb, group_size=group)
+    y = f32(M.affine_mm(dev(x)[:, :in_f], w, out_dtype=tdt(ydt)))
+    sync()
+    wd, mag = dequant(packed, sa, ba, code, group)
+    xd = O.bf16_to_f32(x[:, :in_f]).astype(np.float64)
+    compare(y, xd @ wd.T, np.abs(xd) @ mag.T, in_f, ydt)
+
+
+@pytest.mark.parametrize("tokens", [3, 40])
+def test_affine_few_tokens_non_finite(M, tokens):
+    """An infinite activation and one that overflows the unscaled sums give
+    what dequantized weights give; rows without one are untouched."""
+    print(f"affine few, non-finite T={tokens}", flush=True)
+    packed, sa, ba, code, ts, tb = affine_operand("afi", 40, 256, 64, "bf16")
+    x = O.bf16_to_f32(O.normal_bf16(f"afi.x.{tokens}", (tokens, 256)))
+    x[0, 70] = np.inf
+    x[1, 3] = 3e38  # 3e38 * 15 overflows; times a scale of about 0.01 it does not
+    xb = O.f32_to_bf16(x)
+    w = M.AffineWeights(dev(packed), ts, tb, group_size=64)
+    y = f32(M.affine_mm(dev(xb), w, out_dtype=tdt("f32")))
+    sync()
+    wd, mag = dequant(packed, sa, ba, code, 64)
+    xd = O.bf16_to_f32(xb).astype(np.float64)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = (xd[:, None, :] * wd[None]).sum(-1)
+    np.testing.assert_array_equal(y[0], ref[0].astype(np.float32))
+    ok = np.abs(ref[1:]) < 3e38
+    got = np.where(ok, y[1:], 0).astype(np.float64)
+    compare(got, np.where(ok, ref[1:], 0), np.abs(xd[1:]) @ mag.T, 256, "f32")
