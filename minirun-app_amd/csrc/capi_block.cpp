@@ -554,6 +554,29 @@ mr_status mr_affine_gather_matmul(const void* x, mr_dtype x_dtype, int32_t token
     g.y_stride_row = 1;
     g.y_stride_token = g.out_rows;
     g.force_generic = !aligned16(w->packed);
+    if (x_dtype == MR_BF16 && mr::skinny_routed_better(pairs, experts)) {
+        // each expert's tokens together, on MFMA
+        mr::ProjGemmParams q{};
+        q.x = (const uint16_t*)x;
+        q.ldx = x_stride;
+        q.packed = w->packed;
+        q.scales = w->scales;
+        q.biases = w->biases;
+        q.scale_dtype = scale_code(w->scale_dtype);
+        q.group = w->group;
+        q.bits = w->bits;
+        q.y = y;
+        q.ldy = w->out_features;
+        q.y_f32 = y_dtype == MR_F32;
+        q.M = tokens;
+        q.N = (int)w->out_features;
+        q.K = (int)w->in_features;
+        const mr::SkinnyRoute r{rhs_indices, (int32_t)pairs, experts_per_token, (int32_t)experts};
+        if (mr::skinny_routed_ok(q, r)) {
+            const hipError_t e = mr::launch_skinny_routed(q, r, (hipStream_t)stream);
+            return e == hipSuccess ? MR_OK : hip_fail(e, "affine gather matmul launch");
+        }
+    }
     const hipError_t e = mr::launch_affine_gemv(g, (hipStream_t)stream);
     return e == hipSuccess ? MR_OK : hip_fail(e, "affine gather matmul launch");
 }

@@ -110,3 +110,36 @@ def test_affine_few_tokens_non_finite(M, tokens):
     ok = np.abs(ref[1:]) < 3e38
     got = np.where(ok, y[1:], 0).astype(np.float64)
     compare(got, np.where(ok, ref[1:], 0), np.abs(xd[1:]) @ mag.T, 256, "f32")
+
+
+@pytest.mark.parametrize("tokens,experts,per_token,out_f,in_f,group,sdt,ydt", [
+    (8, 4, 2, 40, 192, 64, "bf16", "f32"),     # four tokens an expert, odd groups, ragged rows
+    (33, 2, 1, 6, 64, 64, "f16", "bf16"),      # more than 16 tokens an expert
+    (40, 8, 4, 64, 1152, 128, "f32", "f32"),
+    (700, 16, 6, 34, 128, 64, "bf16", "bf16"),  # 4200 pairs: two scans
+])
+@pytest.mark.parametrize("bad", [False, True])
+def test_gather_few_tokens_an_expert(M, tokens, experts, per_token, out_f, in_f, group, sdt, ydt, bad):
+    """Routed experts; with `bad`, some ids are out of range (zeros) and one
+    expert has no token."""
+    print(f"gather few T={tokens} E={experts} k={per_token} [{out_f}, {in_f}] g={group} {sdt} {ydt} bad={bad}", flush=True)
+    import torch
+
+    packed, sa, ba, code, ts, tb = affine_operand(f"gf.{experts}.{out_f}.{in_f}", experts * out_f, in_f, group, sdt)
+    rng = np.random.default_rng(tokens * 7 + experts)
+    ids = rng.integers(1 if bad else 0, experts, (tokens, per_token)).astype(np.int32)
+    if bad:
+        ids[::3, 0] = -1
+        ids[1::5, -1] = experts
+    x = O.normal_bf16(f"gf.x.{tokens}.{in_f}", (tokens, in_f))
+    w = M.AffineWeights(dev(packed).reshape(experts, out_f, -1), ts.reshape(experts, out_f, -1),
+                        tb.reshape(experts, out_f, -1), group_size=group)
+    y = f32(M.affine_gather_mm(dev(x), w, torch.from_numpy(ids).cuda(), out_dtype=tdt(ydt)))
+    sync()
+    wd, mag = (a.reshape(experts, out_f, in_f) for a in dequant(packed, sa, ba, code, group))
+    xd = O.bf16_to_f32(x).astype(np.float64)
+    ref, m = np.zeros((tokens, per_token, out_f)), np.zeros((tokens, per_token, out_f))
+    for e in range(experts):
+        t, j = np.nonzero(ids == e)
+        ref[t, j], m[t, j] = xd[t] @ wd[e].T, np.abs(xd[t]) @ mag[e].T
+    compare(y, ref, m, in_f, ydt)
