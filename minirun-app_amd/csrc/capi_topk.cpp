@@ -50,7 +50,7 @@ mr_status mr_indexer_scores(const void* queries, mr_dtype q_dtype, int32_t seq, 
     p.H = heads;
     p.D = dim;
     p.T = n_keys;
-    const hipError_t e = mr::launch_indexer_scores(p, (hipStream_t)stream);
+    const hipError_t e = mr::launch_indexer_scores(p, mrc::cu_count(), (hipStream_t)stream);
     return e == hipSuccess ? MR_OK : hip_fail(e, "lightning-index scores launch");
 }
 

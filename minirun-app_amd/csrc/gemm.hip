@@ -63,13 +63,6 @@ __device__ __forceinline__ int pg_slot(int r, int c) {
     return r * 4 + (c ^ ((r >> 2) & 3));
 }
 
-// DMA of 4 bytes per lane (lane i lands at lds_dst_wave_base + 4 i); the
-// same wait rules as dma16_off
-__device__ __forceinline__ void dma4_off(const void* sbase, uint32_t voff, const void* lds_dst_wave_base) {
-    const uint32_t m0 = (uint32_t)(uintptr_t)lds_dst_wave_base;
-    asm volatile("global_load_lds_dword %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(m0) : "memory");
-}
-
 __device__ __forceinline__ float scale_value(uint32_t bits, int dtype) {
     return dtype == 0 ? __uint_as_float(bits << 16) : (dtype == 1 ? f16_bits_to_f32((uint16_t)bits) : __uint_as_float(bits));
 }

@@ -172,6 +172,13 @@ __device__ __forceinline__ void dma16_off(const void* sbase, uint32_t voff, cons
     asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(m0) : "memory");
 }
 
+// DMA of 4 bytes per lane (lane i lands at lds_dst_wave_base + 4 i); the
+// same wait rules as dma16_off
+__device__ __forceinline__ void dma4_off(const void* sbase, uint32_t voff, const void* lds_dst_wave_base) {
+    const uint32_t m0 = (uint32_t)(uintptr_t)lds_dst_wave_base;
+    asm volatile("global_load_lds_dword %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(m0) : "memory");
+}
+
 // Raw (stride 0) buffer resource over `bytes` bytes from `base`: a load at a
 // byte offset at or past `bytes` returns zeros.  Word 3 holds the gfx9 data
 // format the memory-to-register loads expect (32-bit, no swizzle).

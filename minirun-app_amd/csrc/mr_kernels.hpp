@@ -343,7 +343,7 @@ struct IndexerParams {
     uint32_t k_bytes;
 };
 bool indexer_mfma_ok(const IndexerParams& p);
-hipError_t launch_indexer_scores(const IndexerParams& p, hipStream_t st);
+hipError_t launch_indexer_scores(const IndexerParams& p, int cu_count, hipStream_t st);
 
 // ---------------------------------------------------------------- dense projections
 // y[t][j] = sum_i x_eff[t, xvec(j)][i] * W[wrow(j)][i], W [rows][in] bf16 or

@@ -124,3 +124,34 @@ def test_scores_feed_the_selection(M):
     st, exp = O.topk_select(got.cpu().numpy(), 2048, 4, 131071, 7)
     assert st == O.OK
     np.testing.assert_array_equal(sel.cpu().numpy(), exp)
+
+
+@pytest.mark.parametrize("S,H,T,w_dtype", [
+    (1537, 16, 1, "f32"),     # one key; runs of 3 tokens, a short last one
+    (801, 64, 257, "f32"),    # one key in the second 256-key block
+    (1600, 32, 255, "bf16"),
+    (900, 48, 320, "bf16"),   # a wave's 64 keys, then waves without any
+])
+def test_many_tokens_are_the_bits_of_few(M, S, H, T, w_dtype):
+    """Runs of tokens over 256 keys against the same tokens 32 at a time (one
+    workgroup per token and 128 keys); the first and last against the oracle."""
+    import torch
+
+    print(f"indexer runs S={S} H={H} T={T} weights {w_dtype}", flush=True)
+    q, k, w = inputs(f"r{S}.{H}.{T}", S, H, 128, T)
+    q = q.copy()
+    q[S // 2, 3, 5] = 0x7FC0  # a NaN query stays in its token's row
+    qp = np.zeros((S, H, 136), np.uint16)
+    qp[:, :, :128] = q
+    dq, dk = bf16_dev(qp)[:, :, :128], bf16_dev(k)
+    dw = bf16_dev(O.f32_to_bf16(w)) if w_dtype == "bf16" else f32_dev(w)
+    out = torch.full((S, T + 3), 7.0, dtype=torch.float32, device="cuda")
+    M.lightning_index_scores(dq, dk, dw, out=out[:, :T])
+    parts = torch.cat([M.lightning_index_scores(dq[i:i + 32], dk, dw[i:i + 32]) for i in range(0, S, 32)])
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    np.testing.assert_array_equal(got[:, :T], parts.cpu().numpy())
+    assert (got[:, T:] == 7).all() and np.isnan(got[S // 2, :T]).all()
+    for i in (0, S - 1):
+        ref = O.indexer_scores(O.bf16_to_f32(q[i:i + 1]), O.bf16_to_f32(k), w[i:i + 1])
+        check(got[i:i + 1, :T], ref, f"indexer-run-{i}")
