@@ -7,8 +7,8 @@
 // `visible`.  Exact: the order is a total order on (score, key id) and
 // floats are compared, never combined.
 //
-// One workgroup per row (1024 threads, or 256 for rows of at most 1024
-// keys); thread t holds keys j NT + t (j < KPT) in registers as 48-bit
+// Rows of at most 1024 keys are sorted whole (topk_sort_kernel).  Longer ones:
+// one workgroup of 1024 threads per row; thread t holds keys j NT + t (j < KPT) in registers as 48-bit
 // composites (order-reversing 32-bit image of the score << 16 | key id), so
 // every composite is distinct and ascending composite order is the
 // reference's order (descending score, ties by ascending key id):
@@ -77,7 +77,7 @@ __device__ __forceinline__ uint32_t block_scan_incl(uint32_t v, uint32_t* sh) {
 
 constexpr int TK_BINS = 2048;
 constexpr unsigned long long TK_NONE = ~0ull;  // padding: past every composite
-// Rows ranked by 1024 threads take the compacted path when the first digit's
+// Rows take the compacted path when the first digit's
 // cut bin holds at most TK_CAND keys: the keys above the cut go straight to
 // the selected list and only the cut bin's keys take the remaining digits.
 constexpr int TK_CAND = 4096;
@@ -188,10 +188,12 @@ __device__ void wave_sort(unsigned long long (&x)[EPT], int wsize) {
 // elements EPT t .. EPT t + EPT-1 in registers.  Each wave sorts its 64 EPT
 // elements (wave_sort), then runs of 64 EPT, 128 EPT, ... merge pairwise
 // through LDS: each output position finds its split by a merge-path binary
-// search.  On return x[e] is element EPT t + e of the sorted order; comp
-// holds the last merge's input.
+// search.  On return x[e] is element EPT t + e of the sorted order, if that
+// is below `limit` (the merges leave out what comes later: the first `limit`
+// outputs of a merge come from the first `limit` of each run); comp holds the
+// last merge's input.
 template <int NT, int EPT>
-__device__ void sort_lds(unsigned long long* comp, int npow, unsigned long long (&x)[EPT]) {
+__device__ void sort_lds(unsigned long long* comp, int npow, unsigned long long (&x)[EPT], int limit = INT32_MAX) {
     const int tid = threadIdx.x;
     const bool act = EPT * tid < npow;
 #pragma unroll
@@ -206,12 +208,12 @@ __device__ void sort_lds(unsigned long long* comp, int npow, unsigned long long 
             for (int e = 0; e < EPT; ++e) comp[EPT * tid + e] = x[e];
         }
         __syncthreads();
-        if (act) {
-            const int q0 = EPT * tid;
-            const int base = q0 & ~(2 * run - 1);  // pair start
+        const int q0 = EPT * tid;
+        const int base = q0 & ~(2 * run - 1);  // pair start
+        const int q = q0 - base;               // output position within the pair
+        if (act && q < limit) {
             const unsigned long long* A = comp + base;
             const unsigned long long* B = A + run;
-            const int q = q0 - base;  // output position within the pair
             // i = number of the first q outputs taken from A
             int lo = max(0, q - run), hi = min(q, run);
             while (lo < hi) {
@@ -243,9 +245,8 @@ __global__ void __launch_bounds__(NT) topk_select_kernel(TopkParams p) {
     __shared__ uint32_t scan_sh[NT / 64];
     __shared__ uint32_t pick[3];  // bin, count before it, count in it
     __shared__ unsigned long long comp[TOPK_MAX];
-    constexpr bool FAST = NT == 1024;  // the compacted path (four candidates per thread)
-    constexpr int CPT = FAST ? TK_CAND / NT : 1;
-    __shared__ unsigned long long cand[FAST ? TK_CAND : 1];
+    constexpr int CPT = TK_CAND / NT;  // candidates per thread of the compacted path
+    __shared__ unsigned long long cand[TK_CAND];
     __shared__ int nan_seen;
 
     const int row = blockIdx.x;
@@ -355,7 +356,7 @@ __global__ void __launch_bounds__(NT) topk_select_kernel(TopkParams p) {
         remaining -= pick[1];
         const uint32_t in_bin = pick[2];
         // few keys share the cut bin: rank them apart from the rest
-        if (FAST && pass == 0 && in_bin <= (uint32_t)TK_CAND) {
+        if (pass == 0 && in_bin <= (uint32_t)TK_CAND) {
             cut_count = in_bin;
             fast = true;
             break;
@@ -371,7 +372,7 @@ __global__ void __launch_bounds__(NT) topk_select_kernel(TopkParams p) {
 
     auto composite = [&](int j) { return ((unsigned long long)img[j] << 16) | (uint32_t)(NT * j + tid); };
     static_assert(TK_BINS % 1024 == 0 && TK_CAND >= TOPK_MAX, "bucket arrays");
-    if (FAST && fast) {
+    if (fast) {
         // 2a. keys of bins above the cut bin are all taken: to comp; keys of
         // the cut bin to cand.  One scan places both (counts packed 16:16).
         const uint32_t top = dimg >> 21;
@@ -505,7 +506,7 @@ __global__ void __launch_bounds__(NT) topk_select_kernel(TopkParams p) {
     // scan and a scatter place the buckets, and a key's place inside its
     // bucket is the number of its bucket's keys below it
     bool bucketed = false;
-    if (FAST && k > 1) {  // cand holds the scattered keys (1024-thread rows)
+    if (k > 1) {  // cand holds the scattered keys
         uint32_t* cnt_b = hist[0];
         uint32_t* cur_b = hist[1];
         uint32_t mn = 0xffffffffu, mx = 0u;
@@ -598,6 +599,71 @@ __global__ void __launch_bounds__(NT) topk_select_kernel(TopkParams p) {
     if (p.slices > 1) {
         if (tid == 0) p.slice_nan[row * p.slices + slice] = nan_seen;
         return;
+    }
+    if (tid == 0) {
+        p.nan_flags[row] = nan_seen;
+        if (p.status_direct) *p.status_direct = nan_seen ? 5 /* MR_NONFINITE */ : 0;
+    }
+}
+
+// Rows of at most 1024 ranked keys: the whole row is sorted, with no
+// selection before it.  What bounds it: the VALU work of the sort (a row's
+// scores are 4 KB), with the latency of LDS and barriers hidden by the eight
+// workgroups a CU holds (8 KB of LDS each; the radix select before a sort of
+// half the keys took 24 KB more and about fifteen barriers).  Keys past
+// `visible` all compare as -infinity and are emitted as -1, so without a NaN
+// (which may order below -infinity) only the visible keys are sorted and the
+// rest of the output is -1.
+//
+// Measured with the status launch, radix select of the row by 256 threads ->
+// now: 4001 rows x 1000 keys at 4 rows to a key, top 512 106 -> 57 us, top 8
+// 54 -> 54 us; 1024 x 1024, all 41 -> 23 us; one row of 1000 keys, top 512 14.4
+// -> 13.2 us.
+constexpr int TK_SORT_NT = 256, TK_SORT_KEYS = 4 * TK_SORT_NT;
+
+__global__ void __launch_bounds__(TK_SORT_NT) topk_sort_kernel(TopkParams p) {
+    constexpr int NT = TK_SORT_NT;
+    __shared__ __attribute__((aligned(16))) unsigned long long comp[TK_SORT_KEYS];
+    const int row = blockIdx.x, tid = threadIdx.x;
+    const float* sr = p.scores + (int64_t)row * p.row_stride;
+    const int visible = p.start_pos == 0 ? (row + 1) / p.ratio : p.available;
+    float f[4];
+    bool nan_here = false;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int key = NT * j + tid;
+        f[j] = sr[min(key, p.cols - 1)];
+        nan_here |= isnan(f[j]);
+    }
+    // NaN anywhere in the row (all columns, as the reference checks the whole matrix)
+    for (int i = TK_SORT_KEYS + tid; i < p.cols; i += NT) nan_here |= isnan(sr[i]);
+    const bool nan_seen = __syncthreads_or(nan_here);
+    const int n = nan_seen ? p.available : min(p.available, visible);  // keys to sort
+    int npow = 4;
+    while (npow < n) npow <<= 1;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int key = NT * j + tid;
+        if (key < npow)
+            comp[key] = key < n ? ((unsigned long long)~ordered_bits(key < visible ? f[j] : -INFINITY) << 16) | (uint32_t)key
+                                : TK_NONE;
+    }
+    __syncthreads();
+    unsigned long long x[4];
+    sort_lds<NT, 4>(comp, npow, x, p.selected);
+    int32_t* orow = p.out + (int64_t)row * p.out_stride;
+    int32_t id[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int key = (int)(uint32_t)(x[e] & 0xffffull);
+        id[e] = 4 * tid + e >= n || key >= visible ? -1 : p.offset + key;
+    }
+    if (((uintptr_t)orow & 15) == 0 && 4 * tid + 4 <= p.selected) {
+        *(i32x4*)(orow + 4 * tid) = i32x4{id[0], id[1], id[2], id[3]};
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (4 * tid + e < p.selected) orow[4 * tid + e] = id[e];
     }
     if (tid == 0) {
         p.nan_flags[row] = nan_seen;
@@ -1515,10 +1581,10 @@ hipError_t launch_topk_select(const TopkParams& p0, void* workspace, int32_t* st
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(topk_spread_finish, dim3((unsigned)p.rows), dim3(1024), 0, st, p);
-    } else if (p.available <= 256 * 4) {
-        // keys per thread: the row's ranked keys in registers
-        hipLaunchKernelGGL((topk_select_kernel<256, 4>), dim3((unsigned)p.rows), dim3(256), 0, st, p);
+    } else if (p.available <= TK_SORT_KEYS) {
+        hipLaunchKernelGGL(topk_sort_kernel, dim3((unsigned)p.rows), dim3(TK_SORT_NT), 0, st, p);
     } else if (p.available <= 1024 * 16) {
+        // keys per thread: the row's ranked keys in registers
         hipLaunchKernelGGL((topk_select_kernel<1024, 16>), dim3((unsigned)p.rows), dim3(1024), 0, st, p);
     } else if (p.available <= TOPK_SLICE) {
         hipLaunchKernelGGL((topk_select_kernel<1024, 32>), dim3((unsigned)p.rows), dim3(1024), 0, st, p);

@@ -222,3 +222,21 @@ def test_spread_ties_full_size(M):
     big[0, :261000] = 0.0
     compare(M, big, 2048, 1, 262143, 0, "relu-262144-mostly-zero")
     compare(M, np.zeros((1, 262144), np.float32), 4096, 1, 262143, 0, "zeros-262144-k4096")
+
+
+@pytest.mark.parametrize("cols", [1, 3, 5, 64, 255, 257, 513, 1023, 1024])
+def test_rows_sorted_whole(M, cols):
+    """Rows of at most 1024 keys: few and all of them, ties, visible -inf
+    before masked keys, NaN of either sign reported."""
+    import torch
+
+    rng = np.random.default_rng(cols)
+    for top_k in sorted({1, max(1, cols // 2), cols}):
+        s = np.round(rng.normal(size=(cols, cols)) * 3).astype(np.float32)
+        s[s < -4] = -np.inf
+        compare(M, s, top_k, 1, 0, 5, "sorted whole")
+        compare(M, s[:1], top_k, 1, cols - 1, 0, "sorted whole, one row")
+        s[0, cols // 2], s[cols // 2, 0] = np.float32(np.nan), -np.float32(np.nan)
+        st = torch.zeros(1, dtype=torch.int32, device="cuda")
+        M.lightning_select(dev(s), top_k, 1, 0, 5, check=False, status=st)
+        assert int(st.item()) == 5
