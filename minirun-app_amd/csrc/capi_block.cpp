@@ -395,7 +395,7 @@ mr_status mr_affine_matmul(const void* x, mr_dtype x_dtype, int32_t tokens, int6
         q.N = (int)w->out_features;
         q.K = (int)w->in_features;
         const bool tiles = tokens >= mr::PROJ_GEMM_MIN_TOKENS && mr::proj_gemm_ok(q);
-        if (mr::skinny_gemm_ok(q) && (!tiles || mr::skinny_gemm_better(q.N, q.M, true, mrc::cu_count()))) {
+        if (mr::skinny_gemm_ok(q) && (!tiles || mr::skinny_gemm_better(q.N, q.M, q.K, true, mrc::cu_count()))) {
             const hipError_t e = mr::launch_skinny_gemm(q, mrc::cu_count(), (hipStream_t)stream);
             return e == hipSuccess ? MR_OK : hip_fail(e, "affine matmul launch");
         }
@@ -438,7 +438,7 @@ mr_status mr_linear(const void* x, mr_dtype x_dtype, int32_t tokens, int64_t x_s
         q.N = (int)w->out_features;
         q.K = (int)w->in_features;
         const bool tiles = tokens >= mr::PROJ_GEMM_MIN_TOKENS && mr::proj_gemm_ok(q);
-        if (mr::skinny_gemm_ok(q) && (!tiles || mr::skinny_gemm_better(q.N, q.M, false, mrc::cu_count()))) {
+        if (mr::skinny_gemm_ok(q) && (!tiles || mr::skinny_gemm_better(q.N, q.M, q.K, false, mrc::cu_count()))) {
             const hipError_t e = mr::launch_skinny_gemm(q, mrc::cu_count(), (hipStream_t)stream);
             return e == hipSuccess ? MR_OK : hip_fail(e, "linear launch");
         }
@@ -1071,7 +1071,7 @@ mr_status proj_rows_stacked(const void* x, int32_t tokens, int64_t x_stride, con
         rows += q[i].N;
     }
     // a call each where the few-token tiles are faster than the stack's
-    if (stack && !(few && mr::skinny_gemm_better(rows, tokens, w[0]->kind == MR_PROJ_AFFINE, mrc::cu_count()))) {
+    if (stack && !(few && mr::skinny_gemm_better(rows, tokens, q[0].K, w[0]->kind == MR_PROJ_AFFINE, mrc::cu_count()))) {
         const hipError_t e = mr::launch_proj_gemm_stack(q, n, mrc::cu_count(), (hipStream_t)stream);
         return e == hipSuccess ? MR_OK : hip_fail(e, "stacked projection launch");
     }

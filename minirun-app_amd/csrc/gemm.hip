@@ -5,7 +5,8 @@
 // bits 4j..4j+3, one scale and bias per `group` inputs).  fp32 accumulation;
 // y bf16 or f32.
 //
-// Affine weights are dequantized per k-tile into LDS, w = fp32(scale * q +
+// Affine weights in groups of a multiple of 64 go to affine_gemm.hip, which
+// takes one MFMA per product.  Others are dequantized per k-tile into LDS, w = fp32(scale * q +
 // bias) (exact product, one rounding: the affineDequantize value), and
 // carried as two bf16 operands hi = bf16(w), lo = bf16(w - hi): x is bf16,
 // so x . hi + x . lo on two MFMAs misses x . w by at most 2^-18 |w| per
@@ -443,6 +444,9 @@ hipError_t launch_proj_gemm_stack(const ProjGemmParams* segs, int n, int cu_coun
             ps.tile_end[i] = INT32_MAX;
         }
     }
+    bool groups64 = true;
+    for (int i = 0; i < n; ++i) groups64 = groups64 && affine_gemm_ok(segs[i]) && segs[i].scale_dtype == segs[0].scale_dtype;
+    if (groups64) return launch_affine_gemm(ps, cu_count, st);
     // 256-row tiles when they alone fill the GPU, else 128
     const bool big = (int64_t)((segs[0].M + 255) / 256) * tiles >= cu_count;
     if (segs[0].packed) return big ? launch_y<256, true>(ps, st) : launch_y<128, true>(ps, st);

@@ -209,12 +209,17 @@ bool proj_gemm_ok(const ProjGemmParams& p);  // shapes, alignment and formats th
 hipError_t launch_proj_gemm(const ProjGemmParams& p, int cu_count, hipStream_t st);
 // n entries with one M, all dense or all affine, one output dtype; each proj_gemm_ok
 hipError_t launch_proj_gemm_stack(const ProjGemmParams* segs, int n, int cu_count, hipStream_t st);
+// its affine entries in groups of a multiple of 64 (affine_gemm.hip): every
+// entry proj_gemm_ok and affine_gemm_ok, one scale dtype; N tiles of 256
+bool affine_gemm_ok(const ProjGemmParams& p);
+hipError_t launch_affine_gemm(const ProjGemmStack& ps, int cu_count, hipStream_t st);
+double affine_gemm_cost(int64_t n, int m, int k, int cus);  // us, of n rows in all
 
 // ---------------------------------------------------------------- projections of a few tokens
 // The same product for a few tokens (skinny.hip); affine weights in groups
 // that are a multiple of 64.
 bool skinny_gemm_ok(const ProjGemmParams& p);
-bool skinny_gemm_better(int64_t n, int m, bool affine, int cus);  // than launch_proj_gemm
+bool skinny_gemm_better(int64_t n, int m, int k, bool affine, int cus);  // than launch_proj_gemm
 hipError_t launch_skinny_gemm(const ProjGemmParams& p, int cu_count, hipStream_t st);
 // Routed: pair i (token i / per_token) reads expert ids[i]'s N weight rows of
 // the stacked affine weight and writes y row i; zeros for an id out of range.

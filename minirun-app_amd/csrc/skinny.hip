@@ -38,24 +38,12 @@
 // what those give.
 #include <algorithm>
 
+#include "affine_tiles.hpp"
 #include "mr_kernels.hpp"
 
 namespace mr {
 
 namespace {
-
-// byte offsets outside every buffer (host check: buffers under 2^30 bytes), of
-// a lane's row and of a k-block past the row's end; their sum is outside too
-constexpr uint32_t SK_OOB_ROW = 0x40000000u, SK_OOB_K = 0x80000000u;
-
-// the resource in scalar registers (its inputs are uniform, but may have been
-// computed in vector registers)
-__device__ __forceinline__ i32x4 uniform_rsrc(const void* base, uint32_t bytes) {
-    i32x4 r = buffer_rsrc(base, bytes);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) r[i] = __builtin_amdgcn_readfirstlane(r[i]);
-    return r;
-}
 
 // row tile and token block of this workgroup: consecutive workgroups go to
 // the 8 XCDs in turn
@@ -196,43 +184,6 @@ __global__ void __launch_bounds__(64 * NW) skinny_dense_kernel(ProjGemmParams p,
 }
 
 // ---------------------------------------------------------------- 4-bit affine
-// eight nibbles of a word as bf16 0..15, in their order
-__device__ __forceinline__ bf16x8 nibbles_bf16(uint32_t w) {
-    const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;  // nibbles 0,2,4,6 / 1,3,5,7
-    const uint32_t a = __builtin_amdgcn_perm(hi, lo, 0x05010400u), b = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
-    const u32x4 v = {__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(a, 512.f, false)),
-                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(a, 512.f, true)),
-                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 512.f, false)),
-                     __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 512.f, true))};
-    return __builtin_bit_cast(bf16x8, v);
-}
-
-template <int SDT>
-__device__ __forceinline__ float sk_scale(uint32_t v) {
-    return SDT == 0 ? __uint_as_float(v << 16) : (SDT == 1 ? f16_bits_to_f32((uint16_t)v) : __uint_as_float(v));
-}
-
-// one output from dequantized weights, in order
-template <int SDT>
-__device__ __forceinline__ float sk_affine_dot(const uint16_t* x, const uint32_t* packed, const void* scales,
-                                               const void* biases, int K, int group) {
-    float acc = 0.f;
-#pragma unroll 1
-    for (int i = 0; i < K; ++i) {
-        const int g = i / group;
-        const float s = sk_scale<SDT>(SDT == 2 ? ((const uint32_t*)scales)[g] : ((const uint16_t*)scales)[g]);
-        const float b = sk_scale<SDT>(SDT == 2 ? ((const uint32_t*)biases)[g] : ((const uint16_t*)biases)[g]);
-        const float qv = (float)((packed[i >> 3] >> (4 * (i & 7))) & 15u);
-        acc = fmaf(bf16_bits_to_f32(x[i]), add_rn(mul_rn(s, qv), b), acc);
-    }
-    return acc;
-}
-
-__device__ __forceinline__ void dma4_buf(i32x4 rsrc, uint32_t voff, const void* lds_dst_wave_base) {
-    const uint32_t m0 = (uint32_t)(uintptr_t)lds_dst_wave_base;
-    asm volatile("buffer_load_dword %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "{m0}"(m0) : "memory");
-}
-
 constexpr int SK_SCAN = 4096;  // routed: pairs per scan
 
 // Ring entry: two groups (128 k); W [16 RT rows][64 B] (chunk c of row r in
@@ -550,18 +501,19 @@ int dense_rt(int64_t n, int m, int cus) {
 
 }  // namespace
 
-// Against gemm.hip's tiles, both in rounds of one workgroup per CU.  Dense: a
-// unit of dense_cost takes 1.65 ns per k (52 us at 12288 x 7168, 64 tokens),
-// a round of 128-row tiles 17.5 ns per k (128 us there).  Affine: a round of
-// 32 rows x 64 tokens takes 2.7 ns per k (44 us at K = 16384), a round of
-// 128-row tiles 40 ns (661 us).
-bool skinny_gemm_better(int64_t n, int m, bool affine, int cus) {
+// Against the 128-row tiles, both in rounds of one workgroup per CU.  Dense
+// (gemm.hip): a unit of dense_cost takes 1.65 ns per k (52 us at 12288 x 7168,
+// 64 tokens), a round of tiles 17.5 ns per k (128 us there).  Affine
+// (affine_gemm.hip): a round of 32 rows x 64 tokens takes 2.25 ns per k and 3.5
+// us (7168 x 16384: 128 tokens 81 us, there 194; 500 tokens 290, there 209;
+// 24576 x 1536: 64 tokens 24, there 25, 300 tokens 104, there 52).
+bool skinny_gemm_better(int64_t n, int m, int k, bool affine, int cus) {
     if (m < PROJ_GEMM_MIN_TOKENS) return true;
-    const int64_t tiles = (int64_t)((m + 127) / 128) * ((n + 255) / 256), rounds = (tiles + cus - 1) / cus;
     if (affine) {
         const int64_t wgs = (int64_t)((n + 31) / 32) * ((m + 63) / 64);
-        return (double)((wgs + cus - 1) / cus) * 2.7 < 40. * rounds;
+        return (double)((wgs + cus - 1) / cus) * (k * 2.25e-3 + 3.5) < affine_gemm_cost(n, m, k, cus);
     }
+    const int64_t tiles = (int64_t)((m + 127) / 128) * ((n + 255) / 256), rounds = (tiles + cus - 1) / cus;
     return dense_cost(n, m, dense_rt(n, m, cus), cus) * 1.65 < 17.5 * rounds;
 }
 

@@ -1,5 +1,5 @@
 """Projections of a few tokens (mr_linear, mr_affine_matmul, 2 to about 100
-tokens) and routed experts (mr_affine_gather_matmul) on MFMA, at the edges of
+tokens; 4-bit also many) and routed experts (mr_affine_gather_matmul) on MFMA, at the edges of
 their tiles: 16 tokens, 16 to 48 weight rows, 32 (dense) or 128 (4-bit) k per
 wave and ring entry, 8 waves over K.
 
@@ -89,13 +89,35 @@ def test_affine_few_tokens(M, tokens, out_f, in_f, group, sdt, x_pad, ydt):
     compare(y, xd @ wd.T, np.abs(xd) @ mag.T, in_f, ydt)
 
 
-@pytest.mark.parametrize("tokens", [3, 40])
-def test_affine_few_tokens_non_finite(M, tokens):
+@pytest.mark.parametrize("tokens,out_f,in_f,group,sdt,x_pad,ydt", [
+    (1990, 2056, 64, 64, "f32", 0, "f32"),      # one group: 3 of 4 iterations past the end; ragged tiles both ways
+    (2000, 2056, 192, 64, "f16", 8, "bf16"),    # an odd group count
+    (1985, 2304, 1152, 128, "f32", 0, "f32"),   # one scale for two groups
+    (700, 6000, 1088, 64, "bf16", 0, "f32"),    # 17 groups: scales on both halves of a dword
+    (330, 6000, 1088, 64, "bf16", 16, "bf16"),  # tiles of 64 tokens
+    (321, 6008, 832, 64, "f16", 0, "f32"),      # the same, 13 groups
+    (385, 6000, 1536, 192, "f32", 0, "f32"),    # three groups a scale
+])
+def test_affine_many_tokens(M, tokens, out_f, in_f, group, sdt, x_pad, ydt):
+    """Tiles of 128 or 64 tokens x 256 weight rows (affine_gemm.hip)."""
+    print(f"affine many T={tokens} [{out_f}, {in_f}] g={group} scales={sdt} pad={x_pad} y={ydt}", flush=True)
+    packed, sa, ba, code, ts, tb = affine_operand(f"am.{out_f}.{in_f}", out_f, in_f, group, sdt)
+    x = O.normal_bf16(f"am.x.{tokens}.{in_f}", (tokens, in_f + x_pad))
+    w = M.AffineWeights(dev(packed), ts, tb, group_size=group)
+    y = f32(M.affine_mm(dev(x)[:, :in_f], w, out_dtype=tdt(ydt)))
+    sync()
+    wd, mag = dequant(packed, sa, ba, code, group)
+    xd = O.bf16_to_f32(x[:, :in_f]).astype(np.float64)
+    compare(y, xd @ wd.T, np.abs(xd) @ mag.T, in_f, ydt)
+
+
+@pytest.mark.parametrize("tokens,out_f,in_f", [(3, 40, 256), (40, 40, 256), (2000, 2056, 192), (330, 6000, 1088)])
+def test_affine_non_finite(M, tokens, out_f, in_f):
     """An infinite activation and one that overflows the unscaled sums give
     what dequantized weights give; rows without one are untouched."""
-    print(f"affine few, non-finite T={tokens}", flush=True)
-    packed, sa, ba, code, ts, tb = affine_operand("afi", 40, 256, 64, "bf16")
-    x = O.bf16_to_f32(O.normal_bf16(f"afi.x.{tokens}", (tokens, 256)))
+    print(f"affine, non-finite T={tokens} [{out_f}, {in_f}]", flush=True)
+    packed, sa, ba, code, ts, tb = affine_operand(f"afi.{out_f}", out_f, in_f, 64, "bf16")
+    x = O.bf16_to_f32(O.normal_bf16(f"afi.x.{tokens}", (tokens, in_f)))
     x[0, 70] = np.inf
     x[1, 3] = 3e38  # 3e38 * 15 overflows; times a scale of about 0.01 it does not
     xb = O.f32_to_bf16(x)
@@ -105,11 +127,12 @@ def test_affine_few_tokens_non_finite(M, tokens):
     wd, mag = dequant(packed, sa, ba, code, 64)
     xd = O.bf16_to_f32(xb).astype(np.float64)
     with np.errstate(invalid="ignore", over="ignore"):
-        ref = (xd[:, None, :] * wd[None]).sum(-1)
+        ref = xd @ wd.T
+        ref[0] = (xd[0] * wd).sum(-1)
     np.testing.assert_array_equal(y[0], ref[0].astype(np.float32))
     ok = np.abs(ref[1:]) < 3e38
     got = np.where(ok, y[1:], 0).astype(np.float64)
-    compare(got, np.where(ok, ref[1:], 0), np.abs(xd[1:]) @ mag.T, 256, "f32")
+    compare(got, np.where(ok, ref[1:], 0), np.abs(xd[1:]) @ mag.T, in_f, "f32")
 
 
 @pytest.mark.parametrize("tokens,experts,per_token,out_f,in_f,group,sdt,ydt", [
