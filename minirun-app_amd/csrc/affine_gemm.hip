@@ -25,8 +25,9 @@
 // weight is unpacked by one wave only, in registers, and each x is read from
 // LDS by four waves.  The two halves' sums meet in LDS at the end.
 // An iteration takes 128 k (both halves' group): its x, packed words and scales
-// come by DMA while the one before is used, with one barrier.  v_mfma_f32_32x32x16_bf16, A = x (row = token), B = W (column =
-// weight row): a lane holds one weight row, so its scale is one register.
+// come by DMA while the one before is used, with one barrier.
+// v_mfma_f32_32x32x16_bf16, A = x (row = token), B = W (column = weight row): a
+// lane holds one weight row, so its scale is one register.
 // Within a group the k order is the packed words' own: lane half l / 32 takes
 // words 4 (l / 32) .. + 3, and x chunks to match.
 //

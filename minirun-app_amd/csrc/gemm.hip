@@ -6,9 +6,9 @@
 // y bf16 or f32.
 //
 // Affine weights in groups of a multiple of 64 go to affine_gemm.hip, which
-// takes one MFMA per product.  Others are dequantized per k-tile into LDS, w = fp32(scale * q +
-// bias) (exact product, one rounding: the affineDequantize value), and
-// carried as two bf16 operands hi = bf16(w), lo = bf16(w - hi): x is bf16,
+// takes one MFMA per product.  Others are dequantized per k-tile into LDS, w =
+// fp32(scale * q + bias) (exact product, one rounding: the affineDequantize
+// value), and carried as two bf16 operands hi = bf16(w), lo = bf16(w - hi): x is bf16,
 // so x . hi + x . lo on two MFMAs misses x . w by at most 2^-18 |w| per
 // product, where a single bf16 weight (2^-9 |w|) would put outputs of the
 // 4-bit projections outside a 1e-2 + 2e-2 |y| bar.

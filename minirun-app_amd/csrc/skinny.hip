@@ -199,9 +199,12 @@ constexpr int SK_SCAN = 4096;  // routed: pairs per scan
 // (token, slot) pairs, up to SK_SCAN pairs at a time, and takes them 16 TT at
 // a time; expert index `experts` stands for the ids out of range, whose
 // outputs are zeros.  768 x 2048, 128 experts, 8 per token: 200 tokens 223 ->
-// 50 us, 64 tokens 67 -> 39 us; 4 waves and 16 tokens per workgroup, so
-// that four of them share a CU: a workgroup is a chain of waits (ids, rows,
-// sums), and 8 waves or 32 tokens each were slower.
+// 53 us, 64 tokens 67 -> 39 us.  2 waves and 16 tokens per workgroup, so that
+// seven of them share a CU: a workgroup is a chain of waits (ids, rows, sums),
+// and its waves' shares of a short K are even (4 waves -> 2: 2048 x 768, 200
+// tokens 76 -> 58 us, 1024 x 640 36 -> 28; 768 x 2048 55 -> 53; 1408 x 2048, 512
+// tokens 111 -> 113).  8 waves, 32 tokens or 128 rows each were slower, 64 rows
+// with 4 waves between.
 template <int RT, int TT, int S, int SDT, bool ROUTED, int NW>
 __global__ void __launch_bounds__(64 * NW) skinny_affine_kernel(ProjGemmParams p, SkinnyRoute route, int blocks) {
     static_assert(RT <= 2, "one DMA of scales per entry");
@@ -537,7 +540,7 @@ hipError_t launch_skinny_gemm(const ProjGemmParams& p, int cu_count, hipStream_t
 bool skinny_routed_better(int64_t pairs, int64_t experts) { return pairs >= 2 * experts; }
 
 hipError_t launch_skinny_routed(const ProjGemmParams& p, const SkinnyRoute& route, hipStream_t st) {
-    return launch_affine_sdt<2, 1, 1, true, 4>(p, route, st);
+    return launch_affine_sdt<2, 1, 1, true, 2>(p, route, st);
 }
 
 }  // namespace mr
