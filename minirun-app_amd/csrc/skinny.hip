@@ -271,11 +271,16 @@ __global__ void __launch_bounds__(64 * NW) skinny_affine_kernel(ProjGemmParams p
         auto issue = [&](int i, int slot) {
             char* ent = ring + slot * ENTRY;
             issue_w(i, ent);
-            const uint32_t o = i < n ? 256u * (uint32_t)(w + NW * i) : SK_OOB_K;
+            const int blk = w + NW * i;
+            const uint32_t o = i < n ? 256u * (uint32_t)blk : SK_OOB_K;
+            // an odd last group: the entry's second half is past the row's
+            // end, where the next row or padding may hold a NaN
+            const bool half = 2 * blk + 1 == G;
+            const uint32_t o2[2] = {half && lr >= 8 ? SK_OOB_K : o, half && lr < 8 ? SK_OOB_K : o};  // u < 2, u >= 2
 #pragma unroll
             for (int t = 0; t < TT; ++t)
 #pragma unroll
-                for (int u = 0; u < 4; ++u) dma16_buf(xres, xo[t][u] + o, ent + XOFF + 4096 * t + 1024 * u);
+                for (int u = 0; u < 4; ++u) dma16_buf(xres, xo[t][u] + o2[u >> 1], ent + XOFF + 4096 * t + 1024 * u);
         };
         f32x4 part[RT][TT];
 #pragma unroll

@@ -166,3 +166,34 @@ def test_gather_few_tokens_an_expert(M, tokens, experts, per_token, out_f, in_f,
         t, j = np.nonzero(ids == e)
         ref[t, j], m[t, j] = xd[t] @ wd[e].T, np.abs(xd[t]) @ mag[e].T
     compare(y, ref, m, in_f, ydt)
+
+
+@pytest.mark.parametrize("in_f", [64, 192, 1088])  # odd group counts: the last 128 k end in the next row
+@pytest.mark.parametrize("tokens,experts", [(2, 0), (16, 0), (40, 0), (330, 0), (33, 4)])
+def test_rows_do_not_see_what_follows_them(M, tokens, experts, in_f):
+    """A row's outputs are the same bits whatever its padding and the other
+    tokens hold, NaN and infinities among it."""
+    import torch
+
+    out_f = 6000 if tokens > 64 else 40
+    print(f"affine, a row beside NaN T={tokens} E={experts} [{out_f}, {in_f}]", flush=True)
+    packed, _, _, _, ts, tb = affine_operand(f"anb.{experts}.{out_f}.{in_f}", max(1, experts) * out_f, in_f, 64, "bf16")
+    x = O.bf16_to_f32(O.normal_bf16(f"anb.x.{tokens}.{in_f}", (tokens, in_f + 64)))
+    odd = x.copy()
+    odd[:, in_f:] = np.nan
+    odd[1::3, :64] = np.nan
+    odd[2::3, :8] = np.inf
+    ids = torch.from_numpy(np.random.default_rng(5).integers(0, max(1, experts), (tokens, 2)).astype(np.int32)).cuda()
+
+    def call(a):
+        v = dev(O.f32_to_bf16(a))[:, :in_f]
+        if experts:
+            w = M.AffineWeights(dev(packed).reshape(experts, out_f, -1), ts.reshape(experts, out_f, -1),
+                                tb.reshape(experts, out_f, -1), group_size=64)
+            return M.affine_gather_mm(v, w, ids, out_dtype=tdt("f32"))
+        return M.affine_mm(v, M.AffineWeights(dev(packed), ts, tb, group_size=64), out_dtype=tdt("f32"))
+
+    y, z = f32(call(x)), f32(call(odd))
+    sync()
+    np.testing.assert_array_equal(z[0::3], y[0::3])
+    assert np.isnan(z[1::3]).all()
