@@ -35,8 +35,8 @@
 // with ones and writes the three bf16 parts per (token, group) to LDS; after
 // four iterations every wave adds its rows' biases times them.
 //
-// Outputs that are not finite are computed again from dequantized weights, as
-// in skinny.hip.  Rows past T or N read zeros and are not stored.
+// Outputs that are not finite are computed again from dequantized weights, by
+// the wave that holds them, as in skinny.hip.  Rows past T or N read zeros and are not stored.
 #include <algorithm>
 
 #include "affine_tiles.hpp"
@@ -312,17 +312,27 @@ __global__ void __launch_bounds__(AG_THREADS) affine_gemm_kernel(ProjGemmStack p
             const int i = v >> 5, j = (v >> 4) & 1, e = v & 15;
             const int m = 32 * (OWN + i) + 8 * (e >> 2) + 4 * h + (e & 3), nn = 64 * wc + 32 * j + r32;
             const float y = acc[OWN + i][j][e] + ((const float*)&ex[(((w ^ 4) * (MI / 2) + i) * 8 + j * 4 + (e >> 2)) * 64 + l])[e & 3];
-            if (!(fabsf(y) < INFINITY)) again |= 1ull << v;
-            if (m < toks && nn < rows) store(m, nn, y);
+            if (m >= toks || nn >= rows) continue;
+            if (fabsf(y) < INFINITY)
+                store(m, nn, y);
+            else
+                again |= 1ull << v;
         }
-        while (again) {
-            const int v = __builtin_ctzll(again);
-            again &= again - 1;
-            const int i = v >> 5, j = (v >> 4) & 1, e = v & 15;
-            const int m = 32 * (OWN + i) + 8 * (e >> 2) + 4 * h + (e & 3), nn = 64 * wc + 32 * j + r32;
-            if (m < toks && nn < rows)
-                store(m, nn, sk_affine_dot<SDT>(xb + m * p.ldx, (const uint32_t*)(wbase + (int64_t)nn * wrow),
-                                                sbase + (int64_t)nn * srow, bbase + (int64_t)nn * srow, p.K, p.group));
+        if (!__ballot(again != 0)) return;
+        int finite = -1;
+        // token by token: lane half b of bit (i, j, e) holds row 32 j + its lane
+        // for token 32 i + 8 (e / 4) + 4 b + e % 4
+#pragma unroll 1
+        for (int t = 0; t < 16 * MI; ++t) {
+            const int v = (t & ~31) + 4 * ((t & 31) >> 3) + (t & 3), up = 32 * ((t >> 2) & 1);
+            const uint64_t lo = __ballot((again >> v) & 1), hi = __ballot((again >> (v + 16)) & 1);
+            const uint64_t which = ((lo >> up) & 0xffffffffull) | ((hi >> up) << 32);
+            if (!which) continue;
+            const int m = 32 * OWN + t;
+            const int64_t r0 = 64 * wc;
+            const float y = sk_affine_again<SDT>(which, xb + m * p.ldx, wbase + r0 * wrow, sbase + r0 * srow, bbase + r0 * srow,
+                                                 wrow, srow, p.K, p.group, finite);
+            if ((which >> l) & 1) store(m, 64 * wc + l, y);
         }
     };
     if (kh == 0)

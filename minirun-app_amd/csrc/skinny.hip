@@ -34,8 +34,8 @@
 // by v_cvt_scalef32_pk_bf16_fp8: the e4m3 codes 0..15 are q * 2^-9 (0..7
 // subnormal), and the scale 2^9 makes them q.  An output that is not finite
 // that way (an infinite activation, or a sum that overflows without its
-// scale) is computed again from dequantized weights, one by one, so it holds
-// what those give.
+// scale) is computed again from dequantized weights, so it holds what those
+// give.
 #include <algorithm>
 
 #include "affine_tiles.hpp"
@@ -206,7 +206,7 @@ constexpr int SK_SCAN = 4096;  // routed: pairs per scan
 // tokens 111 -> 113).  8 waves, 32 tokens or 128 rows each were slower, 64 rows
 // with 4 waves between.
 template <int RT, int TT, int S, int SDT, bool ROUTED, int NW>
-__global__ void __launch_bounds__(64 * NW) skinny_affine_kernel(ProjGemmParams p, SkinnyRoute route, int blocks) {
+__global__ void __launch_bounds__(64 * NW, ROUTED ? 3 : 1) skinny_affine_kernel(ProjGemmParams p, SkinnyRoute route, int blocks) {
     static_assert(RT <= 2, "one DMA of scales per entry");
     extern __shared__ __attribute__((aligned(16))) char lds[];
     constexpr int NI = RT + 4 * TT + 2, XOFF = 1024 * RT, SOFF = XOFF + 4096 * TT, ENTRY = SOFF + 512;
@@ -355,20 +355,34 @@ __global__ void __launch_bounds__(64 * NW) skinny_affine_kernel(ProjGemmParams p
         wait_vmcnt<0>();
         sk_reduce<RT, TT, NW>(lds, tot, [&](int r, int t, int lane, f32x4 v) {
             const int nn = 16 * r + (lane & 15);
-            if (nn >= rows) return;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int m = 16 * t + 4 * (lane >> 4) + i;
-                if (m >= toks) break;
-                float y = v[i];
-                if (!(fabsf(y) < INFINITY))
-                    y = sk_affine_dot<SDT>(xb + xrow_of(m) * p.ldx, (const uint32_t*)(wbase + (int64_t)nn * wrow),
-                                           sbase + (int64_t)nn * srow, bbase + (int64_t)nn * srow, p.K, p.group);
-                const int64_t o = yrow_of(m) * p.ldy + n0 + nn;
+            auto store = [&](int m, int row, float y) {
+                const int64_t o = yrow_of(m) * p.ldy + n0 + row;
                 if (p.y_f32)
                     ((float*)p.y)[o] = y;
                 else
                     ((uint16_t*)p.y)[o] = f32_to_bf16_bits(y);
+            };
+            uint32_t again = 0;  // values that are not finite
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int m = 16 * t + 4 * (lane >> 4) + i;
+                if (nn >= rows || m >= toks) continue;
+                if (fabsf(v[i]) < INFINITY)
+                    store(m, nn, v[i]);
+                else
+                    again |= 1u << i;
+            }
+            if (!__ballot(again)) return;
+            int finite = -1;
+#pragma unroll 1
+            for (int i = 0; i < 16; ++i) {
+                const uint64_t lanes = __ballot((again >> (i & 3)) & 1u), which = (lanes >> (16 * (i >> 2))) & 0xffffu;
+                if (!which) continue;
+                const int m = 16 * t + i;
+                const float y = sk_affine_again<SDT>(which, xb + xrow_of(m) * p.ldx, wbase + (int64_t)(16 * r) * wrow,
+                                                     sbase + (int64_t)(16 * r) * srow, bbase + (int64_t)(16 * r) * srow,
+                                                     wrow, srow, p.K, p.group, finite);
+                if ((which >> lane) & 1) store(m, 16 * r + lane, y);
             }
         });
     };

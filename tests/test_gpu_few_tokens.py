@@ -197,3 +197,78 @@ def test_rows_do_not_see_what_follows_them(M, tokens, experts, in_f):
     sync()
     np.testing.assert_array_equal(z[0::3], y[0::3])
     assert np.isnan(z[1::3]).all()
+
+
+@pytest.mark.parametrize("tokens,out_f,in_f,sdt", [
+    (14, 40, 256, "bf16"), (70, 37, 16384, "f32"), (2000, 2056, 192, "f16"), (330, 6000, 1088, "bf16"),
+])
+def test_affine_non_finite_rows(M, tokens, out_f, in_f, sdt):
+    """Rows with NaN, infinities (one, of both signs, everywhere) or sums that
+    overflow unscaled, against what dequantized weights give; one weight row is
+    positive throughout, one has an infinite group."""
+    print(f"affine, non-finite rows T={tokens} [{out_f}, {in_f}] {sdt}", flush=True)
+    import torch
+
+    packed, sa, ba, code, ts, tb = affine_operand(f"afr.{out_f}.{in_f}", out_f, in_f, 64, sdt)
+    top = {"bf16": 0x7FFF, "f16": 0x7FFF, "f32": None}[sdt]
+    ba = ba.copy()
+    ba[0] = np.abs(ba[0]) if top is None else ba[0] & top  # weights of row 0: all >= 0
+    ba[5, -1] = {"bf16": 0x7F80, "f16": 0x7C00, "f32": np.inf}[sdt]
+    tb = torch.from_numpy(ba).view({"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[sdt]).cuda()
+    x = O.bf16_to_f32(O.normal_bf16(f"afr.x.{tokens}.{in_f}", (tokens, in_f))).copy()
+    last = in_f - 1
+    x[1::7, 0::in_f - 1] = np.nan
+    x[2::7, last // 2] = np.inf
+    x[3::7, 3], x[3::7, last] = np.inf, -np.inf
+    x[4::7] = np.inf
+    x[5::7, 1:130] = -np.inf  # more infinities than are taken one by one
+    x[6::7, 9] = 3e38
+    xb = O.f32_to_bf16(x)
+    y = f32(M.affine_mm(dev(xb), M.AffineWeights(dev(packed), ts, tb, group_size=64), out_dtype=tdt("f32")))
+    sync()
+    wd, mag = dequant(packed, sa, ba, code, 64)
+    xd = O.bf16_to_f32(xb).astype(np.float64)
+    for kind in range(7):
+        rows = np.arange(kind, tokens, 7)[:6]
+        with np.errstate(invalid="ignore", over="ignore"):
+            ref = np.stack([(xd[r] * wd).sum(-1) for r in rows])
+            m = np.stack([(np.abs(xd[r]) * mag).sum(-1) for r in rows])
+        fin = np.isfinite(ref)
+        np.testing.assert_array_equal(np.where(fin, 0, y[rows]), np.where(fin, 0, ref).astype(np.float32), str(kind))
+        compare(np.where(fin, y[rows], 0), np.where(fin, ref, 0), np.where(fin, m, 0), in_f, "f32")
+        assert fin.any() == (kind in (0, 6))
+    assert (y[4::7, 0] == np.inf).all() and (y[5::7, 0] == -np.inf).all()
+
+
+@pytest.mark.parametrize("tokens", [13, 300])
+def test_non_finite_rows_cost_little(M, tokens):
+    """Activations that are NaN, or hold an infinity in every row, take a small
+    multiple of the time of finite ones (1.2 to 4.4 measured; an output at a
+    time per lane it was 200 to 1000)."""
+    import torch
+
+    out_f, in_f = 7168, 16384
+    print(f"affine, time of non-finite rows T={tokens} [{out_f}, {in_f}]", flush=True)
+    packed = torch.randint(-2 ** 31, 2 ** 31 - 1, (out_f, in_f // 8), device="cuda").to(torch.int32)
+    s = (torch.randn(out_f, in_f // 64, device="cuda").abs() * 0.01).to(torch.bfloat16)
+    w = M.AffineWeights(packed, s, -7.5 * s, group_size=64)
+    x = torch.randn(tokens, in_f, device="cuda").to(torch.bfloat16)
+    one = x.clone()
+    one[:, 77] = float("inf")
+
+    def us(v):
+        M.affine_mm(v, w)
+        best = float("inf")
+        for _ in range(3):
+            a, b = torch.cuda.Event(True), torch.cuda.Event(True)
+            a.record()
+            M.affine_mm(v, w)
+            M.affine_mm(v, w)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 500)
+        return best
+
+    t = us(x)
+    for v, name in ((torch.full_like(x, float("nan")), "nan"), (one, "inf")):
+        assert us(v) < 12 * t, name
