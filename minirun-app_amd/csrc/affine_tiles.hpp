@@ -55,7 +55,8 @@ constexpr int SK_INFS = 64;
 template <int SDT>
 __device__ float sk_affine_again(uint64_t rows, const uint16_t* x, const char* packed, const char* scales,
                                  const char* biases, uint32_t wrow, uint32_t srow, int K, int group, int& finite) {
-    const int l = threadIdx.x & 63;
+    int l = threadIdx.x & 63;
+    asm volatile("" : "+v"(l));  // no address of this is worth a register outside
     const bool mine = (rows >> l) & 1;
     auto scale = [&](const char* p, int g) {
         return sk_scale<SDT>(SDT == 2 ? ((const uint32_t*)p)[g] : ((const uint16_t*)p)[g]);
@@ -122,7 +123,7 @@ __device__ float sk_affine_again(uint64_t rows, const uint16_t* x, const char* p
         const uint32_t* wj = (const uint32_t*)(packed + (int64_t)j * wrow);
         const char *sj = scales + (int64_t)j * srow, *bj = biases + (int64_t)j * srow;
         float d = 0.f;
-#pragma unroll 2
+#pragma unroll 1
         for (int k = 8 * l; k < K; k += 512) {
             const u32x4 v = *(const u32x4*)(x + k);
             const uint32_t word = wj[k >> 3];

@@ -554,7 +554,7 @@ mr_status mr_affine_gather_matmul(const void* x, mr_dtype x_dtype, int32_t token
     g.y_stride_row = 1;
     g.y_stride_token = g.out_rows;
     g.force_generic = !aligned16(w->packed);
-    if (x_dtype == MR_BF16 && mr::skinny_routed_better(pairs, experts)) {
+    if (x_dtype == MR_BF16 && mr::skinny_routed_better(pairs, experts, w->out_features, w->in_features)) {
         // each expert's tokens together, on MFMA
         mr::ProjGemmParams q{};
         q.x = (const uint16_t*)x;
@@ -571,9 +571,9 @@ mr_status mr_affine_gather_matmul(const void* x, mr_dtype x_dtype, int32_t token
         q.M = tokens;
         q.N = (int)w->out_features;
         q.K = (int)w->in_features;
-        const mr::SkinnyRoute r{rhs_indices, (int32_t)pairs, experts_per_token, (int32_t)experts};
+        const mr::SkinnyRoute r{rhs_indices, (int32_t)pairs, experts_per_token, (int32_t)experts, 0, 0};
         if (mr::skinny_routed_ok(q, r)) {
-            const hipError_t e = mr::launch_skinny_routed(q, r, (hipStream_t)stream);
+            const hipError_t e = mr::launch_skinny_routed(q, r, mrc::cu_count(), (hipStream_t)stream);
             return e == hipSuccess ? MR_OK : hip_fail(e, "affine gather matmul launch");
         }
     }

@@ -227,10 +227,13 @@ hipError_t launch_skinny_gemm(const ProjGemmParams& p, int cu_count, hipStream_t
 struct SkinnyRoute {
     const int32_t* ids;
     int32_t pairs, per_token, experts;
+    // set by the launcher: pairs of a window, log2, and workgroups (of each row
+    // tile) for an expert's windows after its first
+    int32_t shift, slots;
 };
 bool skinny_routed_ok(const ProjGemmParams& p, const SkinnyRoute& route);
-bool skinny_routed_better(int64_t pairs, int64_t experts);  // than a GEMV per pair
-hipError_t launch_skinny_routed(const ProjGemmParams& p, const SkinnyRoute& route, hipStream_t st);
+bool skinny_routed_better(int64_t pairs, int64_t experts, int64_t n, int64_t k);  // than a GEMV per pair
+hipError_t launch_skinny_routed(const ProjGemmParams& p, const SkinnyRoute& route, int cu_count, hipStream_t st);
 
 hipError_t launch_prefill_attn(const PrefillAttnParams& p, hipStream_t st);
 

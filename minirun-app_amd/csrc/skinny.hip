@@ -74,7 +74,8 @@ __device__ __forceinline__ void sk_reduce(char* lds, const f32x4 (&acc)[RT][TT],
         for (int n = 1; n < NW; n *= 2)
 #pragma unroll
             for (int k = 0; k + n < NW; k += 2 * n) v[k] += v[k + n];
-        emit((i >> 6) / TT, (i >> 6) % TT, i & 63, v[0]);
+        const int rt = __builtin_amdgcn_readfirstlane(i >> 6);
+        emit(rt / TT, rt % TT, i & 63, v[0]);
     }
 }
 
@@ -184,7 +185,131 @@ __global__ void __launch_bounds__(64 * NW) skinny_dense_kernel(ProjGemmParams p,
 }
 
 // ---------------------------------------------------------------- 4-bit affine
-constexpr int SK_SCAN = 4096;  // routed: pairs per scan
+constexpr int SK_IDS = 32;            // routed: ids per thread and scan
+constexpr int SK_WINDOW_MAX_LOG2 = 9;  // pairs per workgroup
+constexpr int SK_MAX_EXPERTS = 3072;   // bins in the ring of sk_find_window
+
+// Routed, pairs lo .. hi - 1 of expert e, as the scans find them, into `list`
+// (expert index `experts`: the ids out of range); how many there are.  Every
+// workgroup that asks for an expert finds its pairs in one order, so the windows
+// of an expert do not overlap.  sums: an int per wave.
+//
+// A scan costs its instructions: each of the workgroups looks at every id, four
+// instructions an id here (with a ballot and a count per 64 ids it was a fifth
+// of the whole call at 4096 pairs).
+template <int NW>
+__device__ __forceinline__ int sk_collect(const SkinnyRoute& route, int e, int lo, int hi, int32_t* list, int32_t* sums) {
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    // ids from e, or all from `experts` up as unsigned numbers
+    const uint32_t span = e == route.experts ? 0u - (uint32_t)e : 1u;
+    int seen = 0;  // of the expert's pairs, before this scan
+#pragma unroll 1
+    for (int base = 0; base < route.pairs && seen < hi; base += 64 * NW * SK_IDS) {
+        // a wave takes `per` runs of 64 pairs, one after the other
+        const int left = min(route.pairs - base, 64 * NW * SK_IDS), per = (left + 64 * NW - 1) / (64 * NW);
+        const int first = 64 * per * w + l;
+        const __amdgpu_buffer_rsrc_t ids =
+            __builtin_amdgcn_make_buffer_rsrc((void*)(route.ids + base), 0, 4 * left, 0x00020000);
+        uint32_t id[SK_IDS], hit = 0;  // bit u: pair first + 64 u is the expert's
+#pragma unroll
+        for (int u0 = 0; u0 < SK_IDS; u0 += 8)
+            if (u0 < per) {
+#pragma unroll
+                for (int u = u0; u < u0 + 8; ++u) id[u] = __builtin_amdgcn_raw_buffer_load_b32(ids, 4 * first + 256 * u, 0, 0);
+            }
+#pragma unroll
+        for (int u0 = SK_IDS - 8; u0 >= 0; u0 -= 8)
+            if (u0 < per) {
+#pragma unroll
+                for (int u = u0 + 7; u >= u0; --u) hit = (hit << 1) | (id[u] - (uint32_t)e < span ? 1u : 0u);
+            }
+        const int valid = min(per, (left - first + 63) / 64);  // past it: zeros, or another wave's pairs
+        hit &= valid <= 0 ? 0u : ~0u >> (32 - valid);
+        const int mine = __popc(hit);
+        int incl = mine;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int up = __shfl_up(incl, d);
+            if (l >= d) incl += up;
+        }
+        if (l == 63) sums[w] = incl;
+        __syncthreads();
+        int r = seen - lo + incl - mine;
+#pragma unroll
+        for (int k = 0; k < NW; ++k) {
+            const int c = __builtin_amdgcn_readfirstlane(sums[k]);
+            if (k < w) r += c;
+            seen += c;
+        }
+        while (hit) {
+            if (r >= 0 && r < hi - lo) list[r] = base + first + 64 * __builtin_ctz(hit);
+            hit &= hit - 1;
+            ++r;
+        }
+        __syncthreads();  // the list is whole; the sums are free
+    }
+    return max(0, min(seen, hi) - lo);
+}
+
+// Routed: the o-th window, of 2^shift pairs, after the first of each expert:
+// {expert, which of its windows}, or {-1, ..} past the last.  bins: an int per
+// expert and one more; sums: NW + 2.
+template <int NW>
+__device__ __forceinline__ int2 sk_find_window(const SkinnyRoute& route, int o, int32_t* bins, int32_t* sums) {
+    constexpr int NT = 64 * NW;
+    const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, n = route.experts + 1;
+    for (int i = tid; i < n; i += NT) bins[i] = 0;
+    if (tid == 0) sums[NW] = -1;
+    __syncthreads();
+    auto load = [&](int (&id)[8], int base) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) id[u] = route.ids[min(base + NT * u + tid, route.pairs - 1)];
+    };
+    int id[8], next[8];
+    load(id, 0);
+#pragma unroll 1
+    for (int base = 0; base < route.pairs; base += 8 * NT) {
+        if (base + 8 * NT < route.pairs) load(next, base + 8 * NT);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int bin = (int)min((uint32_t)id[u], (uint32_t)route.experts);
+            // lane 0 adds for all lanes of its expert: the ids of a hot one
+            // would be 64 adds to one word, one after the other
+            const bool in = base + NT * u + tid < route.pairs, same = bin == __builtin_amdgcn_readfirstlane(bin);
+            const int n = __popcll(__ballot(in && same));
+            if (in && (!same || l == 0)) atomicAdd(&bins[bin], same ? n : 1);
+            id[u] = next[u];
+        }
+    }
+    __syncthreads();
+    // a thread takes `run` experts one after the other
+    const int run = (n + NT - 1) / NT;
+    int mine = 0;
+    for (int j = tid * run; j < min(n, (tid + 1) * run); ++j) mine += max(0, bins[j] - 1) >> route.shift;
+    int incl = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int up = __shfl_up(incl, d);
+        if (l >= d) incl += up;
+    }
+    if (l == 63) sums[w] = incl;
+    __syncthreads();
+    for (int k = 0; k < w; ++k) incl += sums[k];
+    if (o >= incl - mine && o < incl) {
+        int at = incl - mine, j = tid * run;
+        for (;; ++j) {
+            const int more = max(0, bins[j] - 1) >> route.shift;
+            if (o < at + more) break;
+            at += more;
+        }
+        sums[NW] = j;
+        sums[NW + 1] = o - at + 1;
+    }
+    __syncthreads();
+    const int2 r = make_int2(__builtin_amdgcn_readfirstlane(sums[NW]), __builtin_amdgcn_readfirstlane(sums[NW + 1]));
+    __syncthreads();  // bins and sums are free
+    return r;
+}
 
 // Ring entry: two groups (128 k); W [16 RT rows][64 B] (chunk c of row r in
 // slot c ^ ((r >> 2) & 3)), x [16 TT rows][256 B] (slot c ^ (r % 16)), then per
@@ -195,27 +320,33 @@ constexpr int SK_SCAN = 4096;  // routed: pairs per scan
 // us, 64 tokens 661 -> 44 us; 24576 x 1536, 13 tokens 780 -> 11 us.  One ring
 // entry per wave (S = 1, all 8 waves' entries in flight) is as fast as three.
 //
-// Routed: workgroup (expert, row tile).  It scans the ids for its expert's
-// (token, slot) pairs, up to SK_SCAN pairs at a time, and takes them 16 TT at
-// a time; expert index `experts` stands for the ids out of range, whose
-// outputs are zeros.  768 x 2048, 128 experts, 8 per token: 200 tokens 223 ->
-// 53 us, 64 tokens 67 -> 39 us.  2 waves and 16 tokens per workgroup, so that
-// seven of them share a CU: a workgroup is a chain of waits (ids, rows, sums),
-// and its waves' shares of a short K are even (4 waves -> 2: 2048 x 768, 200
-// tokens 76 -> 58 us, 1024 x 640 36 -> 28; 768 x 2048 55 -> 53; 1408 x 2048, 512
-// tokens 111 -> 113).  8 waves, 32 tokens or 128 rows each were slower, 64 rows
-// with 4 waves between.
+// Routed: workgroup (expert, row tile).  It scans the ids for the first window of
+// its expert's (token, slot) pairs and takes them 16 TT at a time; expert index
+// `experts` stands for the ids out of range, whose outputs are zeros.  Further
+// workgroups take the windows that follow a first one: each counts every expert's
+// pairs and finds every route.slots-th of them, so that a hot expert is no chain
+// of passes.  They cost nothing that could be measured where no expert is hot.
+//
+// 2 waves and 16 tokens, eight workgroups a CU (at most 128 registers: 160 to 180
+// without the bound, and 8 to 40% slower): a workgroup is a chain of waits (ids,
+// rows, sums).  768 x 2048, 128 experts, 8 per token, 200 tokens: 207 us by a GEMV
+// per pair, 46 now; half of the slots on one expert 321 -> 57, all on one 207 ->
+// 53 (318 and 609 when an expert was one workgroup per row tile).  2048 x 768: 247
+// -> 45 us, 256 x 512 of 256 experts, 2048 tokens: 262 -> 45.  4 or 8 waves, 32
+// tokens, 64 or 128 rows each were slower with one workgroup per expert.
 template <int RT, int TT, int S, int SDT, bool ROUTED, int NW>
-__global__ void __launch_bounds__(64 * NW, ROUTED ? 3 : 1) skinny_affine_kernel(ProjGemmParams p, SkinnyRoute route, int blocks) {
+__global__ void __launch_bounds__(64 * NW, ROUTED ? 4 : 1) skinny_affine_kernel(ProjGemmParams p, SkinnyRoute route, int blocks) {
     static_assert(RT <= 2, "one DMA of scales per entry");
     extern __shared__ __attribute__((aligned(16))) char lds[];
     constexpr int NI = RT + 4 * TT + 2, XOFF = 1024 * RT, SOFF = XOFF + 4096 * TT, ENTRY = SOFF + 512;
     static_assert((S - 1) * NI < 64, "vmcnt range");
+    static_assert(!ROUTED || 4 * (SK_MAX_EXPERTS + 1) <= NW * S * ENTRY, "bins");
     const int tid = threadIdx.x, l = tid & 63, q = l >> 4, lr = l & 15;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     int tile, tb = 0, e = 0;
     const int n_tiles = (p.N + 16 * RT - 1) / (16 * RT);
-    if (ROUTED) {
+    int32_t* const list = (int32_t*)(lds + std::max(NW * S * ENTRY, NW * RT * TT * 1024));
+    if constexpr (ROUTED) {
         e = blockIdx.x / n_tiles;
         tile = blockIdx.x - e * n_tiles;
     } else {
@@ -227,37 +358,42 @@ __global__ void __launch_bounds__(64 * NW, ROUTED ? 3 : 1) skinny_affine_kernel(
     const uint32_t wrow = (uint32_t)p.K / 2, srow = (uint32_t)(p.K / p.group) * (SDT == 2 ? 4 : 2);
     const int gpl = p.group / 64;  // 64-groups per scale
     const int n = w < nblk ? (nblk - 1 - w) / NW + 1 : 0;  // this wave's entries
-    const int64_t wr0 = (int64_t)(ROUTED ? min(e, route.experts - 1) : 0) * p.N + n0;
-    const char* wbase = (const char*)p.packed + wr0 * wrow;
-    const char *sbase = (const char*)p.scales + wr0 * srow, *bbase = (const char*)p.biases + wr0 * srow;
-    const i32x4 wres = uniform_rsrc(wbase, (uint32_t)rows * wrow);
-    // (2-byte scales: through the dword that holds the last one)
-    const i32x4 sres = uniform_rsrc(sbase, ((uint32_t)rows * srow + 3u) & ~3u);
-    const i32x4 bres = uniform_rsrc(bbase, ((uint32_t)rows * srow + 3u) & ~3u);
-    uint32_t wo[RT];
-#pragma unroll
-    for (int r = 0; r < RT; ++r) {
-        const int row = 16 * r + (l >> 2);
-        wo[r] = row < rows ? (uint32_t)row * wrow + 16u * ((l & 3) ^ ((l >> 4) & 3)) : SK_OOB_ROW;
-    }
-    // lane l of the scale DMA: row l / 2, group l % 2 of the entry
-    const uint32_t so = (l >> 1) < rows ? (uint32_t)(l >> 1) * srow : SK_OOB_ROW;
-    char* ring = lds + w * S * ENTRY;
-    auto issue_w = [&](int i, char* ent) {
-        const int blk = w + NW * i;
-        const uint32_t o = i < n ? 64u * blk : SK_OOB_K;
-#pragma unroll
-        for (int r = 0; r < RT; ++r) dma16_buf(wres, wo[r] + o, ent + 1024 * r);
-        const int g = min(2 * blk + (l & 1), G - 1);  // a group past the last is not used
-        const uint32_t gs = (uint32_t)(gpl == 1 ? g : g / gpl) * (SDT == 2 ? 4 : 2);
-        const uint32_t sv = i < n ? (so + gs) & ~3u : SK_OOB_K;
-        dma4_buf(sres, sv, ent + SOFF);
-        dma4_buf(bres, sv, ent + SOFF + 256);
+    const char *wbase, *sbase, *bbase;
+    i32x4 wres, sres, bres;
+    auto set_rows = [&](int64_t first) {  // the weight rows of this workgroup: first + n0 ..
+        wbase = (const char*)p.packed + (first + n0) * wrow;
+        sbase = (const char*)p.scales + (first + n0) * srow;
+        bbase = (const char*)p.biases + (first + n0) * srow;
+        wres = uniform_rsrc(wbase, (uint32_t)rows * wrow);
+        // (2-byte scales: through the dword that holds the last one)
+        sres = uniform_rsrc(sbase, ((uint32_t)rows * srow + 3u) & ~3u);
+        bres = uniform_rsrc(bbase, ((uint32_t)rows * srow + 3u) & ~3u);
     };
+    if constexpr (!ROUTED) set_rows(0);
     const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
     f32x4 tot[RT][TT];
     // the products of `toks` tokens: x row and y row of token i from row_of
     auto tokens = [&](int toks, const uint16_t* xb, int64_t xbytes, auto xrow_of, auto yrow_of) {
+        uint32_t wo[RT];
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+            const int row = 16 * r + (l >> 2);
+            wo[r] = row < rows ? (uint32_t)row * wrow + 16u * ((l & 3) ^ ((l >> 4) & 3)) : SK_OOB_ROW;
+        }
+        // lane l of the scale DMA: row l / 2, group l % 2 of the entry
+        const uint32_t so = (l >> 1) < rows ? (uint32_t)(l >> 1) * srow : SK_OOB_ROW;
+        char* ring = lds + w * S * ENTRY;
+        auto issue_w = [&](int i, char* ent) {
+            const int blk = w + NW * i;
+            const uint32_t o = i < n ? 64u * blk : SK_OOB_K;
+#pragma unroll
+            for (int r = 0; r < RT; ++r) dma16_buf(wres, wo[r] + o, ent + 1024 * r);
+            const int g = min(2 * blk + (l & 1), G - 1);  // a group past the last is not used
+            const uint32_t gs = (uint32_t)(gpl == 1 ? g : g / gpl) * (SDT == 2 ? 4 : 2);
+            const uint32_t sv = i < n ? (so + gs) & ~3u : SK_OOB_K;
+            dma4_buf(sres, sv, ent + SOFF);
+            dma4_buf(bres, sv, ent + SOFF + 256);
+        };
         const i32x4 xres = uniform_rsrc(xb, (uint32_t)xbytes);
         // lane l of DMA u: row 4 u + l / 16, slot l % 16, chunk slot ^ (row % 16)
         uint32_t xo[TT][4];
@@ -372,7 +508,7 @@ __global__ void __launch_bounds__(64 * NW, ROUTED ? 3 : 1) skinny_affine_kernel(
                 else
                     again |= 1u << i;
             }
-            if (!__ballot(again)) return;
+            if (__builtin_expect(!__ballot(again), 1)) return;
             int finite = -1;
 #pragma unroll 1
             for (int i = 0; i < 16; ++i) {
@@ -391,45 +527,41 @@ __global__ void __launch_bounds__(64 * NW, ROUTED ? 3 : 1) skinny_affine_kernel(
         tokens(toks, p.x + (int64_t)m0 * p.ldx, ((int64_t)(toks - 1) * p.ldx + p.K) * 2,
                [](int i) { return (int64_t)i; }, [&](int i) { return (int64_t)(m0 + i); });
     } else {
-        constexpr int IDS = SK_SCAN / (64 * NW);  // ids per thread
-        uint16_t* list = (uint16_t*)(lds + std::max(NW * S * ENTRY, NW * RT * TT * 1024));
-        int& count = *(int*)(list + SK_SCAN);
-        for (int base = 0; base < route.pairs; base += SK_SCAN) {
-            int id[IDS];
-#pragma unroll
-            for (int u = 0; u < IDS; ++u) id[u] = route.ids[min(base + u * (64 * NW) + tid, route.pairs - 1)];
-            if (tid == 0) count = 0;
-            __syncthreads();
-            // in no particular order: a token's products do not depend on
-            // its place among the others
-#pragma unroll
-            for (int u = 0; u < IDS; ++u) {
-                const int i = u * (64 * NW) + tid;
-                const bool bad = (uint32_t)id[u] >= (uint32_t)route.experts;
-                if (base + i < route.pairs && (e == route.experts ? bad : id[u] == e))
-                    list[atomicAdd(&count, 1)] = (uint16_t)i;
+        const int32_t* pairs = list + NW;
+        // the first window of expert e; or, past the experts, every
+        // route.slots-th of the windows that follow a first one
+        const bool later = e > route.experts;
+#pragma unroll 1
+        for (int o = e - route.experts - 1;; o += route.slots) {
+            int window = 0;
+            if (later) {
+                const int2 f = sk_find_window<NW>(route, o, (int32_t*)lds, list);
+                if (f.x < 0) return;
+                e = f.x;
+                window = f.y;
             }
-            __syncthreads();
-            const int cnt = count;
+            const int lo = window << route.shift;
+            const int cnt = sk_collect<NW>(route, e, lo, lo + (1 << route.shift), list + NW, list);
+            set_rows((int64_t)min(e, route.experts - 1) * p.N);
+#pragma unroll 1
             for (int i0 = 0; i0 < cnt; i0 += 16 * TT) {
                 const int toks = min(16 * TT, cnt - i0);
                 if (e == route.experts) {
                     for (int i = tid; i < toks * rows; i += 64 * NW) {
-                        const int64_t o = (int64_t)(base + list[i0 + i / rows]) * p.ldy + n0 + i % rows;
+                        const int64_t y = (int64_t)pairs[i0 + i / rows] * p.ldy + n0 + i % rows;
                         if (p.y_f32)
-                            ((float*)p.y)[o] = 0.f;
+                            ((float*)p.y)[y] = 0.f;
                         else
-                            ((uint16_t*)p.y)[o] = 0;
+                            ((uint16_t*)p.y)[y] = 0;
                     }
                 } else {
-                    auto pair = [&](int i) { return base + (int)list[i0 + i]; };
                     tokens(toks, p.x, ((int64_t)(p.M - 1) * p.ldx + p.K) * 2,
-                           [&](int i) { return (int64_t)((uint32_t)pair(i) / (uint32_t)route.per_token); },
-                           [&](int i) { return (int64_t)pair(i); });
-                    __syncthreads();  // the partial sums are read before the ring is written again
+                           [&](int i) { return (int64_t)((uint32_t)pairs[i0 + i] / (uint32_t)route.per_token); },
+                           [&](int i) { return (int64_t)pairs[i0 + i]; });
                 }
+                __syncthreads();  // partial sums and the list are read before they are written again
             }
-            __syncthreads();  // the list and count too
+            if (!later) return;
         }
     }
 }
@@ -455,13 +587,14 @@ hipError_t launch_dense(const ProjGemmParams& p, hipStream_t st) {
 template <int RT, int TT, int S, int SDT, bool ROUTED, int NW>
 hipError_t launch_affine(const ProjGemmParams& p, const SkinnyRoute& route, hipStream_t st) {
     constexpr size_t ring = std::max<size_t>((size_t)NW * S * (1024 * RT + 4096 * TT + 512), (size_t)NW * RT * TT * 1024);
-    constexpr size_t lds = ring + (ROUTED ? SK_SCAN * 2 + 4 : 0);
-    static_assert(lds <= 163840, "LDS");
+    const size_t lds = ring + (ROUTED ? 4 * (NW + std::max(2, 1 << route.shift)) : 0);
+    static_assert(ring + 4 * (NW + (1 << SK_WINDOW_MAX_LOG2)) <= 163840, "LDS");
     const auto kern = skinny_affine_kernel<RT, TT, S, SDT, ROUTED, NW>;
     const hipError_t e = set_lds(kern, lds);
     if (e != hipSuccess) return e;
     const int tiles = (p.N + 16 * RT - 1) / (16 * RT), blocks = (p.M + 16 * TT - 1) / (16 * TT);
-    const unsigned grid = ROUTED ? (unsigned)(tiles * (route.experts + 1)) : (unsigned)((tiles + 7) / 8 * 8 * blocks);
+    const unsigned grid = ROUTED ? (unsigned)(tiles * (route.experts + 1 + route.slots))
+                                 : (unsigned)((tiles + 7) / 8 * 8 * blocks);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * NW), lds, st, p, route, blocks);
     return hipGetLastError();
 }
@@ -493,8 +626,8 @@ bool skinny_gemm_ok(const ProjGemmParams& p) {
 }
 
 bool skinny_routed_ok(const ProjGemmParams& p, const SkinnyRoute& route) {
-    return p.packed && skinny_gemm_ok(p) && (int64_t)p.M * p.ldx * 2 < (1 << 30) && route.pairs <= INT32_MAX - SK_SCAN &&
-           ((int64_t)p.N / 32 + 1) * (route.experts + 1) < INT32_MAX;
+    return p.packed && skinny_gemm_ok(p) && (int64_t)p.M * p.ldx * 2 < (1 << 30) && route.pairs < (1 << 30) &&
+           route.experts < SK_MAX_EXPERTS && ((int64_t)p.N / 32 + 1) * (route.experts + 1 + route.pairs / 16) < (1 << 25);
 }
 
 namespace {
@@ -553,12 +686,31 @@ hipError_t launch_skinny_gemm(const ProjGemmParams& p, int cu_count, hipStream_t
     return rt == 1 ? launch_dense<1, 4, 2, 8>(p, st) : (rt == 2 ? launch_dense<2, 4, 3, 8>(p, st) : launch_dense<3, 4, 2, 8>(p, st));
 }
 
-// A workgroup per expert and row tile pays once an expert has a few tokens; a
-// GEMV per (token, slot) is faster below (128 experts: 128 pairs 20 against 26
-// us, 512 pairs 67 against 39 us)
-bool skinny_routed_better(int64_t pairs, int64_t experts) { return pairs >= 2 * experts; }
+// Than a GEMV per pair.  Pays once an expert has two tokens (128 experts of 768 x
+// 2048, 256 pairs 35 against 31 us, 128 pairs 20 against 27), and once the GEMV,
+// about 4.5 us and 14e12 weights a second, takes longer than a workgroup's chain
+// of waits, 6 to 13 us by K (8 experts of 1408 x 2048, 32 pairs, 92e6 weights:
+// 11.5 against 13.0 us, 40 pairs 17.8 against 13.1; 64 of 512 x 1024, 128 pairs,
+// 67e6: 10.4 against 10.6, with half of them to one expert 9.5 against 13.8, 160
+// pairs 18.2 against 10.7; 256 of 256 x 512, 512 pairs, 67e6: 13.1 against 11.6).
+bool skinny_routed_better(int64_t pairs, int64_t experts, int64_t n, int64_t k) {
+    return pairs >= 2 * experts && (double)pairs * (double)n * (double)k >= 40e6 + 30e3 * (double)k;
+}
 
-hipError_t launch_skinny_routed(const ProjGemmParams& p, const SkinnyRoute& route, hipStream_t st) {
+// Windows of 16 pairs (one pass) up to twice the mean of an expert, so that few
+// experts have a second one; but where the experts alone do not fill the GPU, four
+// workgroups a CU, no more than lets the windows fill it (one expert of 768 x 2048,
+// 512 pairs: 17 us, 62 by the GEMV).  As many workgroups for the windows that
+// follow a first one: two a CU instead of four take 110 us instead of 81 at 2048 x
+// 768 and 200 tokens all on one expert.
+hipError_t launch_skinny_routed(const ProjGemmParams& p, const SkinnyRoute& r, int cu_count, hipStream_t st) {
+    SkinnyRoute route = r;
+    const int tiles = (p.N + 31) / 32;
+    route.shift = 4;
+    while (route.shift < SK_WINDOW_MAX_LOG2 && ((int64_t)route.experts << route.shift) < 2 * (int64_t)route.pairs &&
+           ((int64_t)tiles * route.experts >= 4 * cu_count || ((int64_t)tiles * route.pairs >> (route.shift + 1)) >= 4 * cu_count))
+        ++route.shift;
+    route.slots = std::min(route.pairs >> route.shift, (4 * cu_count + tiles - 1) / tiles);
     return launch_affine_sdt<2, 1, 1, true, 2>(p, route, st);
 }
 

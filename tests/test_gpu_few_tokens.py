@@ -142,9 +142,9 @@ def test_affine_non_finite(M, tokens, out_f, in_f):
     (700, 16, 6, 34, 128, 64, "bf16", "bf16"),  # 4200 pairs: two scans
 ])
 @pytest.mark.parametrize("bad", [False, True])
-def test_gather_few_tokens_an_expert(M, tokens, experts, per_token, out_f, in_f, group, sdt, ydt, bad):
-    """Routed experts; with `bad`, some ids are out of range (zeros) and one
-    expert has no token."""
+def test_gather_few_pairs(M, tokens, experts, per_token, out_f, in_f, group, sdt, ydt, bad):
+    """Routed experts, a GEMV per pair; with `bad`, some ids are out of range
+    (zeros) and one expert has no token."""
     print(f"gather few T={tokens} E={experts} k={per_token} [{out_f}, {in_f}] g={group} {sdt} {ydt} bad={bad}", flush=True)
     import torch
 
@@ -169,13 +169,13 @@ def test_gather_few_tokens_an_expert(M, tokens, experts, per_token, out_f, in_f,
 
 
 @pytest.mark.parametrize("in_f", [64, 192, 1088])  # odd group counts: the last 128 k end in the next row
-@pytest.mark.parametrize("tokens,experts", [(2, 0), (16, 0), (40, 0), (330, 0), (33, 4)])
+@pytest.mark.parametrize("tokens,experts", [(2, 0), (16, 0), (40, 0), (330, 0), (900, 4)])
 def test_rows_do_not_see_what_follows_them(M, tokens, experts, in_f):
     """A row's outputs are the same bits whatever its padding and the other
     tokens hold, NaN and infinities among it."""
     import torch
 
-    out_f = 6000 if tokens > 64 else 40
+    out_f = 400 if experts else (6000 if tokens > 64 else 40)
     print(f"affine, a row beside NaN T={tokens} E={experts} [{out_f}, {in_f}]", flush=True)
     packed, _, _, _, ts, tb = affine_operand(f"anb.{experts}.{out_f}.{in_f}", max(1, experts) * out_f, in_f, 64, "bf16")
     x = O.bf16_to_f32(O.normal_bf16(f"anb.x.{tokens}.{in_f}", (tokens, in_f + 64)))
@@ -272,3 +272,83 @@ def test_non_finite_rows_cost_little(M, tokens):
     t = us(x)
     for v, name in ((torch.full_like(x, float("nan")), "nan"), (one, "inf")):
         assert us(v) < 12 * t, name
+
+
+def routing(kind, tokens, experts, per_token):
+    """ids [tokens, per_token]: uniform; all on one expert; half of the slots on
+    one; counts at the edges of passes of 16 and of windows, the rest on the last
+    expert; or half of them out of range."""
+    rng = np.random.default_rng(tokens + experts)
+    ids = rng.integers(0, experts, (tokens, per_token)).astype(np.int32)
+    if kind == "one":
+        ids[:] = experts - 1
+    elif kind == "half":
+        ids[:, :(per_token + 1) // 2] = experts // 2
+    elif kind == "edges":
+        flat = np.full(tokens * per_token, experts - 1, np.int32)
+        counts = [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 64, 65, 128, 129][:experts - 1]
+        at = np.cumsum([0] + counts)
+        for e, (i, j) in enumerate(zip(at[:-1], at[1:])):
+            flat[i:j] = e
+        ids = rng.permutation(flat).reshape(tokens, per_token)
+    elif kind == "bad":
+        ids[::2] = experts
+        ids[::4, 0] = -2 ** 31
+    return ids
+
+
+@pytest.mark.parametrize("kind", ["uniform", "one", "half", "edges", "bad"])
+@pytest.mark.parametrize("tokens,experts,per_token,out_f,in_f,group,sdt,ydt", [
+    (700, 16, 6, 98, 192, 64, "bf16", "bf16"),   # 4200 pairs: two scans; an odd group count, ragged rows
+    (300, 128, 8, 40, 1152, 128, "f32", "f32"),
+    (700, 3, 6, 70, 192, 64, "f16", "f32"),
+    (4400, 4, 2, 96, 64, 64, "bf16", "f32"),     # more windows of one expert than workgroups for them
+])
+def test_gather_tokens_an_expert_together(M, tokens, experts, per_token, out_f, in_f, group, sdt, ydt, kind):
+    print(f"gather T={tokens} E={experts} k={per_token} [{out_f}, {in_f}] g={group} {sdt} {ydt} {kind}", flush=True)
+    import torch
+
+    packed, sa, ba, code, ts, tb = affine_operand(f"gt.{experts}.{out_f}.{in_f}", experts * out_f, in_f, group, sdt)
+    ids = routing(kind, tokens, experts, per_token)
+    x = O.normal_bf16(f"gt.x.{tokens}.{in_f}", (tokens, in_f))
+    w = M.AffineWeights(dev(packed).reshape(experts, out_f, -1), ts.reshape(experts, out_f, -1),
+                        tb.reshape(experts, out_f, -1), group_size=group)
+    y = f32(M.affine_gather_mm(dev(x), w, torch.from_numpy(ids).cuda(), out_dtype=tdt(ydt)))
+    sync()
+    wd, mag = (a.reshape(experts, out_f, in_f) for a in dequant(packed, sa, ba, code, group))
+    xd = O.bf16_to_f32(x).astype(np.float64)
+    ref, m = np.zeros((tokens, per_token, out_f)), np.zeros((tokens, per_token, out_f))
+    for e in range(experts):
+        t, j = np.nonzero(ids == e)
+        ref[t, j], m[t, j] = xd[t] @ wd[e].T, np.abs(xd[t]) @ mag[e].T
+    compare(y, ref, m, in_f, ydt)
+
+
+def test_a_hot_expert_is_no_chain(M):
+    """200 tokens, 8 slots each, all on one of 128 experts: a small multiple of the
+    time that spread slots take (1.2 measured; 13 with one workgroup per expert
+    and row tile)."""
+    import torch
+
+    experts, out_f, in_f = 128, 768, 2048
+    print(f"gather, time of a hot expert E={experts} [{out_f}, {in_f}]", flush=True)
+    packed = torch.randint(-2 ** 31, 2 ** 31 - 1, (experts, out_f, in_f // 8), device="cuda").to(torch.int32)
+    s = (torch.randn(experts, out_f, in_f // 64, device="cuda").abs() * 0.01).to(torch.bfloat16)
+    w = M.AffineWeights(packed, s, -7.5 * s, group_size=64)
+    x = torch.randn(200, in_f, device="cuda").to(torch.bfloat16)
+    spread = torch.rand(200, experts, device="cuda").topk(8, dim=1).indices.to(torch.int32).contiguous()
+
+    def us(ids):
+        M.affine_gather_mm(x, w, ids)
+        best = float("inf")
+        for _ in range(5):
+            a, b = torch.cuda.Event(True), torch.cuda.Event(True)
+            a.record()
+            for _ in range(10):
+                M.affine_gather_mm(x, w, ids)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 100)
+        return best
+
+    assert us(torch.full_like(spread, 5)) < 4 * us(spread)
