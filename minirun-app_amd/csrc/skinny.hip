@@ -329,10 +329,10 @@ __device__ __forceinline__ int2 sk_find_window(const SkinnyRoute& route, int o, 
 //
 // 2 waves and 16 tokens, eight workgroups a CU (at most 128 registers: 160 to 180
 // without the bound, and 8 to 40% slower): a workgroup is a chain of waits (ids,
-// rows, sums).  768 x 2048, 128 experts, 8 per token, 200 tokens: 207 us by a GEMV
-// per pair, 46 now; half of the slots on one expert 321 -> 57, all on one 207 ->
-// 53 (318 and 609 when an expert was one workgroup per row tile).  2048 x 768: 247
-// -> 45 us, 256 x 512 of 256 experts, 2048 tokens: 262 -> 45.  4 or 8 waves, 32
+// rows, sums).  768 x 2048, 128 experts, 200 tokens of 8 slots, a GEMV per pair ->
+// now: spread 207 -> 45 us, half of the slots on one expert 192 -> 55, all on one
+// 191 -> 48 (318 and 609 when an expert was one workgroup per row tile).  2048 x
+// 768: 247 -> 45; 256 experts of 256 x 512, 2048 tokens 262 -> 45.  4 or 8 waves, 32
 // tokens, 64 or 128 rows each were slower with one workgroup per expert.
 template <int RT, int TT, int S, int SDT, bool ROUTED, int NW>
 __global__ void __launch_bounds__(64 * NW, ROUTED ? 4 : 1) skinny_affine_kernel(ProjGemmParams p, SkinnyRoute route, int blocks) {
@@ -700,9 +700,9 @@ bool skinny_routed_better(int64_t pairs, int64_t experts, int64_t n, int64_t k) 
 // Windows of 16 pairs (one pass) up to twice the mean of an expert, so that few
 // experts have a second one; but where the experts alone do not fill the GPU, four
 // workgroups a CU, no more than lets the windows fill it (one expert of 768 x 2048,
-// 512 pairs: 17 us, 62 by the GEMV).  As many workgroups for the windows that
-// follow a first one: two a CU instead of four take 110 us instead of 81 at 2048 x
-// 768 and 200 tokens all on one expert.
+// 512 pairs: 17 us, 61 by the GEMV).  As many workgroups for the windows that
+// follow a first one: half as many took 1.5 times as long at 2048 x 768, 200 tokens
+// of 8 slots all on one expert (67 us now, 248 by the GEMV).
 hipError_t launch_skinny_routed(const ProjGemmParams& p, const SkinnyRoute& r, int cu_count, hipStream_t st) {
     SkinnyRoute route = r;
     const int tiles = (p.N + 31) / 32;
