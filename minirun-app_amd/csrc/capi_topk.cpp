@@ -116,7 +116,7 @@ mr_status mr_topk_select(const mr_topk_args* a, void* stream) {
     p.out = a->out;
     p.out_stride = a->out_row_stride;
     p.nan_flags = (int32_t*)a->workspace;
-    hipError_t e = mr::launch_topk_select(p, a->workspace, a->status, s);
+    hipError_t e = mr::launch_topk_select(p, a->workspace, a->status, mrc::cu_count(), s);
     if (e != hipSuccess) return hip_fail(e, "top-k selection launch");
     // the reference throws on a NaN score: check on the host unless the
     // caller takes the device status or opts out

@@ -284,7 +284,8 @@ constexpr int TOPK_SPREAD_MAX_ROWS = 8;
 // selection's per-slice arrays; for rows of more than TOPK_SLICE keys the
 // slice flags and two candidate buffers.
 size_t topk_workspace_bytes(int32_t rows, int32_t cols, int32_t selected);
-hipError_t launch_topk_select(const TopkParams& p, void* workspace, int32_t* status, hipStream_t st);
+bool topk_sorts_whole(const TopkParams& p, int cu_count);  // rows of at most 1024 ranked keys: against the radix select
+hipError_t launch_topk_select(const TopkParams& p, void* workspace, int32_t* status, int cu_count, hipStream_t st);
 
 // ---------------------------------------------------------------- affine
 struct AffineDequantParams {

@@ -7,8 +7,9 @@
 // `visible`.  Exact: the order is a total order on (score, key id) and
 // floats are compared, never combined.
 //
-// Rows of at most 1024 keys are sorted whole (topk_sort_kernel).  Longer ones:
-// one workgroup of 1024 threads per row; thread t holds keys j NT + t (j < KPT) in registers as 48-bit
+// Rows of at most 1024 keys of which more than a few are selected are sorted
+// whole (topk_sort_kernel, topk_sorts_whole).  Others: one workgroup per row (1024
+// threads, or 256 for rows of at most 1024 keys); thread t holds keys j NT + t (j < KPT) in registers as 48-bit
 // composites (order-reversing 32-bit image of the score << 16 | key id), so
 // every composite is distinct and ascending composite order is the
 // reference's order (descending score, ties by ascending key id):
@@ -77,7 +78,7 @@ __device__ __forceinline__ uint32_t block_scan_incl(uint32_t v, uint32_t* sh) {
 
 constexpr int TK_BINS = 2048;
 constexpr unsigned long long TK_NONE = ~0ull;  // padding: past every composite
-// Rows take the compacted path when the first digit's
+// Rows ranked by 1024 threads take the compacted path when the first digit's
 // cut bin holds at most TK_CAND keys: the keys above the cut go straight to
 // the selected list and only the cut bin's keys take the remaining digits.
 constexpr int TK_CAND = 4096;
@@ -245,8 +246,9 @@ __global__ void __launch_bounds__(NT) topk_select_kernel(TopkParams p) {
     __shared__ uint32_t scan_sh[NT / 64];
     __shared__ uint32_t pick[3];  // bin, count before it, count in it
     __shared__ unsigned long long comp[TOPK_MAX];
-    constexpr int CPT = TK_CAND / NT;  // candidates per thread of the compacted path
-    __shared__ unsigned long long cand[TK_CAND];
+    constexpr bool FAST = NT == 1024;  // the compacted path (four candidates per thread)
+    constexpr int CPT = FAST ? TK_CAND / NT : 1;
+    __shared__ unsigned long long cand[FAST ? TK_CAND : 1];
     __shared__ int nan_seen;
 
     const int row = blockIdx.x;
@@ -356,7 +358,7 @@ __global__ void __launch_bounds__(NT) topk_select_kernel(TopkParams p) {
         remaining -= pick[1];
         const uint32_t in_bin = pick[2];
         // few keys share the cut bin: rank them apart from the rest
-        if (pass == 0 && in_bin <= (uint32_t)TK_CAND) {
+        if (FAST && pass == 0 && in_bin <= (uint32_t)TK_CAND) {
             cut_count = in_bin;
             fast = true;
             break;
@@ -372,7 +374,7 @@ __global__ void __launch_bounds__(NT) topk_select_kernel(TopkParams p) {
 
     auto composite = [&](int j) { return ((unsigned long long)img[j] << 16) | (uint32_t)(NT * j + tid); };
     static_assert(TK_BINS % 1024 == 0 && TK_CAND >= TOPK_MAX, "bucket arrays");
-    if (fast) {
+    if (FAST && fast) {
         // 2a. keys of bins above the cut bin are all taken: to comp; keys of
         // the cut bin to cand.  One scan places both (counts packed 16:16).
         const uint32_t top = dimg >> 21;
@@ -506,7 +508,7 @@ __global__ void __launch_bounds__(NT) topk_select_kernel(TopkParams p) {
     // scan and a scatter place the buckets, and a key's place inside its
     // bucket is the number of its bucket's keys below it
     bool bucketed = false;
-    if (k > 1) {  // cand holds the scattered keys
+    if (FAST && k > 1) {  // cand holds the scattered keys (1024-thread rows)
         uint32_t* cnt_b = hist[0];
         uint32_t* cur_b = hist[1];
         uint32_t mn = 0xffffffffu, mx = 0u;
@@ -615,10 +617,10 @@ __global__ void __launch_bounds__(NT) topk_select_kernel(TopkParams p) {
 // (which may order below -infinity) only the visible keys are sorted and the
 // rest of the output is -1.
 //
-// Measured with the status launch, radix select of the row by 256 threads ->
-// now: 4001 rows x 1000 keys at 4 rows to a key, top 512 106 -> 57 us, top 8
-// 54 -> 54 us; 1024 x 1024, all 41 -> 23 us; one row of 1000 keys, top 512 14.4
-// -> 13.2 us.
+// Measured with the status launch, radix select of the row by 256 threads -> sort:
+// 4001 rows x 1000 keys at 4 rows to a key, top 512 103 -> 54 us; 1024 x 1024, all
+// 39 -> 22 us; 4096 x 256 at 16 rows to a key, top 8 53 -> 42 us; one row of 1000
+// keys, top 512 12.9 -> 11.9 us.
 constexpr int TK_SORT_NT = 256, TK_SORT_KEYS = 4 * TK_SORT_NT;
 
 __global__ void __launch_bounds__(TK_SORT_NT) topk_sort_kernel(TopkParams p) {
@@ -1541,7 +1543,31 @@ hipError_t merge_rounds(const TopkParams& p, unsigned long long* const* buf, int
 
 }  // namespace
 
-hipError_t launch_topk_select(const TopkParams& p0, void* workspace, int32_t* status, hipStream_t st) {
+// Whether rows of at most 1024 ranked keys are sorted whole.  The sort costs by
+// the visible keys whatever is selected, the radix select by the selected ones
+// and little by the keys.  Radix select -> sort, us: one row of 1000 keys, 64 /
+// 128 / 256 selected 10.0 / 11.1 / 11.6 -> 12.0 / 12.1 / 12.2; one of 130, 32 / 64
+// 8.4 / 10.1 -> 9.9 / 10.0; one of 64, any 6.3 to 10 -> 6.3.  Up to three rows a CU
+// the select waits on latency: 512 rows of up to 512 keys, 16 / 32 / 64 selected
+// 13.3 / 14.7 / 16.0 -> 14.7 / 14.7 / 15.0 (768 rows: 14.3 / 15.8 / 16.5 -> 16.6 /
+// 17.1 / 16.9); of up to 128 keys, 1 / 4 / 8 selected 10.5 / 11.1 / 12.0 -> 11.6 /
+// 11.4 / 11.4.  More rows: 2048 of up to 682 keys, 8 /
+// 16 selected 29.6 / 31.7 -> 30.4 / 30.6, of up to 292 27 to 29 for both; 4000 of
+// up to 1000 keys, 4 / 8 selected 49.2 / 52.0 -> 51.9 / 52.1.
+bool topk_sorts_whole(const TopkParams& p, int cu_count) {
+    const int keys = p.start_pos == 0 ? std::min(p.available, p.rows / p.ratio) : p.available;  // visible to the last row
+    if (keys <= 64) return true;
+    int few;  // the radix select is faster up to here
+    if (p.rows == 1)
+        few = keys > 256 ? 128 : (keys > 128 ? 32 : 16);
+    else if (p.rows <= 3 * cu_count)
+        few = keys > 128 ? (p.rows > 2 * cu_count ? 32 : 16) : 4;
+    else
+        few = keys < 512 ? 0 : (p.rows <= 8 * cu_count ? 8 : 4);
+    return p.selected > few;
+}
+
+hipError_t launch_topk_select(const TopkParams& p0, void* workspace, int32_t* status, int cu_count, hipStream_t st) {
     TopkParams p = p0;
     p.slices = 1;
     p.list_len = p.selected;
@@ -1581,8 +1607,10 @@ hipError_t launch_topk_select(const TopkParams& p0, void* workspace, int32_t* st
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(topk_spread_finish, dim3((unsigned)p.rows), dim3(1024), 0, st, p);
-    } else if (p.available <= TK_SORT_KEYS) {
+    } else if (p.available <= TK_SORT_KEYS && topk_sorts_whole(p, cu_count)) {
         hipLaunchKernelGGL(topk_sort_kernel, dim3((unsigned)p.rows), dim3(TK_SORT_NT), 0, st, p);
+    } else if (p.available <= 256 * 4) {
+        hipLaunchKernelGGL((topk_select_kernel<256, 4>), dim3((unsigned)p.rows), dim3(256), 0, st, p);
     } else if (p.available <= 1024 * 16) {
         // keys per thread: the row's ranked keys in registers
         hipLaunchKernelGGL((topk_select_kernel<1024, 16>), dim3((unsigned)p.rows), dim3(1024), 0, st, p);
