@@ -141,8 +141,9 @@ __global__ void __launch_bounds__(256) indexer_scores_mfma(IndexerParams p) {
 // Measured, the kernel above -> this one, 64 heads, f32 weights: 4001 tokens x
 // 1000 keys 146 -> 69 us, 16384 x 4096 2045 -> 925 us, 1200 x 300 18.4 -> 16.4
 // us; 16 heads, 4001 x 1000 117 -> 23 us.  Fewer than IT_MIN_RUN tokens per
-// workgroup stay above: the keys' registers would be filled for one token
-// (65536 keys, 4 tokens: 11.7 us there, 8 tokens: 18.5 -> 13.2 us here).
+// workgroup stay above: the keys' registers would be filled for one token (one of
+// 196700 keys 10.9 us there, 12.3 here; 65536 keys, 4 tokens 12.7 -> 10.3, 8 tokens
+// 21.6 -> 14.2).
 constexpr int IT_KEYS = 256, IT_NS = 3, IT_MIN_RUN = 2;
 constexpr int it_stage(int ht) { return 16 * ht * 256 + 4 * 256; }
 
@@ -269,15 +270,21 @@ bool indexer_mfma_ok(const IndexerParams& p) {
            (int64_t)p.T * p.k_rs * 2 < (int64_t(1) << 31);
 }
 
+int indexer_run(const IndexerParams& p, int cu_count) {
+    if (!indexer_mfma_ok(p) || !indexer_tokens_ok(p)) return 0;
+    // enough workgroups for the three a CU holds, and no run longer than the call
+    const int64_t blocks = (p.T + IT_KEYS - 1) / IT_KEYS;
+    const int64_t run = std::min<int64_t>(p.S, (p.S * blocks + 3 * cu_count - 1) / (3 * cu_count));
+    return run >= IT_MIN_RUN ? (int)run : 0;
+}
+
 hipError_t launch_indexer_scores(const IndexerParams& q, int cu_count, hipStream_t st) {
     if (q.T == 0) return hipSuccess;
     IndexerParams p = q;
     if (indexer_mfma_ok(p)) {
         p.k_bytes = (uint32_t)((int64_t)(p.T - 1) * p.k_rs * 2 + 256);  // through the last key's 128 dims
-        // tokens per workgroup: enough workgroups for the three a CU holds
-        const int64_t blocks = (p.T + IT_KEYS - 1) / IT_KEYS;
-        const int run = (int)std::max<int64_t>(1, (p.S * blocks + 3 * cu_count - 1) / (3 * cu_count));
-        if (run >= IT_MIN_RUN && indexer_tokens_ok(p)) {
+        const int run = indexer_run(p, cu_count);
+        if (run > 0) {
             switch (p.H / 16) {
                 case 1: return launch_tokens<1>(p, run, st);
                 case 2: return launch_tokens<2>(p, run, st);

@@ -352,6 +352,7 @@ struct IndexerParams {
     uint32_t k_bytes;
 };
 bool indexer_mfma_ok(const IndexerParams& p);
+int indexer_run(const IndexerParams& p, int cu_count);  // tokens per workgroup of the many-token kernel; 0: the other
 hipError_t launch_indexer_scores(const IndexerParams& p, int cu_count, hipStream_t st);
 
 // ---------------------------------------------------------------- dense projections

@@ -131,9 +131,10 @@ def test_scores_feed_the_selection(M):
     (801, 64, 257, "f32"),    # one key in the second 256-key block
     (1600, 32, 255, "bf16"),
     (900, 48, 320, "bf16"),   # a wave's 64 keys, then waves without any
+    (4, 16, 65536, "f32"),    # two tokens a workgroup
 ])
 def test_many_tokens_are_the_bits_of_few(M, S, H, T, w_dtype):
-    """Runs of tokens over 256 keys against the same tokens 32 at a time (one
+    """Runs of tokens over 256 keys against the same tokens 32 (or 2) at a time (one
     workgroup per token and 128 keys); the first and last against the oracle."""
     import torch
 
@@ -147,7 +148,8 @@ def test_many_tokens_are_the_bits_of_few(M, S, H, T, w_dtype):
     dw = bf16_dev(O.f32_to_bf16(w)) if w_dtype == "bf16" else f32_dev(w)
     out = torch.full((S, T + 3), 7.0, dtype=torch.float32, device="cuda")
     M.lightning_index_scores(dq, dk, dw, out=out[:, :T])
-    parts = torch.cat([M.lightning_index_scores(dq[i:i + 32], dk, dw[i:i + 32]) for i in range(0, S, 32)])
+    step = min(32, S // 2)
+    parts = torch.cat([M.lightning_index_scores(dq[i:i + step], dk, dw[i:i + step]) for i in range(0, S, step)])
     torch.cuda.synchronize()
     got = out.cpu().numpy()
     np.testing.assert_array_equal(got[:, :T], parts.cpu().numpy())
