@@ -385,10 +385,13 @@ double affine_gemm_cost(int64_t n, int m, int k, int cus) {
     return std::min(tiles_cost(n_tiles, m, k, 2, cus), tiles_cost(n_tiles, m, k, 4, cus));
 }
 
+int affine_gemm_rows(int64_t n_tiles, int m, int k, int cus) {
+    return tiles_cost(n_tiles, m, k, 4, cus) < tiles_cost(n_tiles, m, k, 2, cus) ? 128 : 64;
+}
+
 hipError_t launch_affine_gemm(const ProjGemmStack& ps, int cu_count, hipStream_t st) {
     const int n_tiles = ps.tile_end[ps.nseg - 1], m = ps.seg[0].M, k = ps.seg[0].K;
-    return tiles_cost(n_tiles, m, k, 4, cu_count) < tiles_cost(n_tiles, m, k, 2, cu_count) ? launch_sdt<4>(ps, st)
-                                                                                             : launch_sdt<2>(ps, st);
+    return affine_gemm_rows(n_tiles, m, k, cu_count) == 128 ? launch_sdt<4>(ps, st) : launch_sdt<2>(ps, st);
 }
 
 }  // namespace mr

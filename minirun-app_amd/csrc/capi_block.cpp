@@ -394,13 +394,11 @@ mr_status mr_affine_matmul(const void* x, mr_dtype x_dtype, int32_t tokens, int6
         q.M = tokens;
         q.N = (int)w->out_features;
         q.K = (int)w->in_features;
-        const bool tiles = tokens >= mr::PROJ_GEMM_MIN_TOKENS && mr::proj_gemm_ok(q);
-        if (mr::skinny_gemm_ok(q) && (!tiles || mr::skinny_gemm_better(q.N, q.M, q.K, true, mrc::cu_count()))) {
-            const hipError_t e = mr::launch_skinny_gemm(q, mrc::cu_count(), (hipStream_t)stream);
-            return e == hipSuccess ? MR_OK : hip_fail(e, "affine matmul launch");
-        }
-        if (tiles) {
-            const hipError_t e = mr::launch_proj_gemm(q, mrc::cu_count(), (hipStream_t)stream);
+        const int cus = mrc::cu_count();
+        const mr::ProjRoute route = mr::proj_route(q, cus);
+        if (route != mr::PROJ_GEMV) {
+            const hipError_t e = route == mr::PROJ_FEW ? mr::launch_skinny_gemm(q, cus, (hipStream_t)stream)
+                                                       : mr::launch_proj_gemm(q, cus, (hipStream_t)stream);
             return e == hipSuccess ? MR_OK : hip_fail(e, "affine matmul launch");
         }
     }
@@ -437,13 +435,11 @@ mr_status mr_linear(const void* x, mr_dtype x_dtype, int32_t tokens, int64_t x_s
         q.M = tokens;
         q.N = (int)w->out_features;
         q.K = (int)w->in_features;
-        const bool tiles = tokens >= mr::PROJ_GEMM_MIN_TOKENS && mr::proj_gemm_ok(q);
-        if (mr::skinny_gemm_ok(q) && (!tiles || mr::skinny_gemm_better(q.N, q.M, q.K, false, mrc::cu_count()))) {
-            const hipError_t e = mr::launch_skinny_gemm(q, mrc::cu_count(), (hipStream_t)stream);
-            return e == hipSuccess ? MR_OK : hip_fail(e, "linear launch");
-        }
-        if (tiles) {
-            const hipError_t e = mr::launch_proj_gemm(q, mrc::cu_count(), (hipStream_t)stream);
+        const int cus = mrc::cu_count();
+        const mr::ProjRoute route = mr::proj_route(q, cus);
+        if (route != mr::PROJ_GEMV) {
+            const hipError_t e = route == mr::PROJ_FEW ? mr::launch_skinny_gemm(q, cus, (hipStream_t)stream)
+                                                       : mr::launch_proj_gemm(q, cus, (hipStream_t)stream);
             return e == hipSuccess ? MR_OK : hip_fail(e, "linear launch");
         }
     }

@@ -427,6 +427,9 @@ bool proj_gemm_ok(const ProjGemmParams& p) {
     return true;
 }
 
+// 256-row tiles when they alone fill the GPU, else 128
+int proj_gemm_rows(int64_t n_tiles, int m, int cu_count) { return (m + 255) / 256 * n_tiles >= cu_count ? 256 : 128; }
+
 hipError_t launch_proj_gemm_stack(const ProjGemmParams* segs, int n, int cu_count, hipStream_t st) {
     if (n < 1 || n > 3) return hipErrorInvalidValue;
     ProjGemmStack ps{};
@@ -447,10 +450,18 @@ hipError_t launch_proj_gemm_stack(const ProjGemmParams* segs, int n, int cu_coun
     bool groups64 = true;
     for (int i = 0; i < n; ++i) groups64 = groups64 && affine_gemm_ok(segs[i]) && segs[i].scale_dtype == segs[0].scale_dtype;
     if (groups64) return launch_affine_gemm(ps, cu_count, st);
-    // 256-row tiles when they alone fill the GPU, else 128
-    const bool big = (int64_t)((segs[0].M + 255) / 256) * tiles >= cu_count;
+    const bool big = proj_gemm_rows(tiles, segs[0].M, cu_count) == 256;
     if (segs[0].packed) return big ? launch_y<256, true>(ps, st) : launch_y<128, true>(ps, st);
     return big ? launch_y<256, false>(ps, st) : launch_y<128, false>(ps, st);
+}
+
+// A GEMV for one token and for what neither takes
+ProjRoute proj_route(const ProjGemmParams& p, int cu_count) {
+    if (p.M <= 1) return PROJ_GEMV;
+    const bool tiles = p.M >= PROJ_GEMM_MIN_TOKENS && proj_gemm_ok(p);
+    if (skinny_gemm_ok(p) && (!tiles || skinny_gemm_better(p.N, p.M, p.K, p.packed != nullptr, cu_count))) return PROJ_FEW;
+    if (!tiles) return PROJ_GEMV;
+    return affine_gemm_ok(p) ? PROJ_GROUP_TILES : PROJ_TILES;
 }
 
 hipError_t launch_proj_gemm(const ProjGemmParams& p, int cu_count, hipStream_t st) {

@@ -206,12 +206,18 @@ struct ProjGemmStack {
 };
 constexpr int PROJ_GEMM_MIN_TOKENS = 64;  // fewer tokens take skinny.hip's tiles or the GEMV kernels
 bool proj_gemm_ok(const ProjGemmParams& p);  // shapes, alignment and formats the kernel takes
+int proj_gemm_rows(int64_t n_tiles, int m, int cu_count);  // rows of its tiles: 256 or 128
+// What a projection of bf16 tokens runs on: a GEMV (affine.hip, linear.hip), the
+// few-token tiles (skinny.hip), gemm.hip's tiles, or affine_gemm.hip's
+enum ProjRoute { PROJ_GEMV, PROJ_FEW, PROJ_TILES, PROJ_GROUP_TILES };
+ProjRoute proj_route(const ProjGemmParams& p, int cu_count);
 hipError_t launch_proj_gemm(const ProjGemmParams& p, int cu_count, hipStream_t st);
 // n entries with one M, all dense or all affine, one output dtype; each proj_gemm_ok
 hipError_t launch_proj_gemm_stack(const ProjGemmParams* segs, int n, int cu_count, hipStream_t st);
 // its affine entries in groups of a multiple of 64 (affine_gemm.hip): every
 // entry proj_gemm_ok and affine_gemm_ok, one scale dtype; N tiles of 256
 bool affine_gemm_ok(const ProjGemmParams& p);
+int affine_gemm_rows(int64_t n_tiles, int m, int k, int cus);  // tokens of its tiles: 128 or 64
 hipError_t launch_affine_gemm(const ProjGemmStack& ps, int cu_count, hipStream_t st);
 double affine_gemm_cost(int64_t n, int m, int k, int cus);  // us, of n rows in all
 

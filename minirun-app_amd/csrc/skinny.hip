@@ -566,6 +566,17 @@ __global__ void __launch_bounds__(64 * NW, ROUTED ? 4 : 1) skinny_affine_kernel(
     }
 }
 
+// Token tiles of 16 per workgroup
+int token_tiles(int m) { return m <= 16 ? 1 : (m <= 32 ? 2 : 4); }
+
+int64_t workgroups(int64_t n, int m, int rt) {
+    const int tt = token_tiles(m);
+    return ((n + 16 * rt - 1) / (16 * rt) + 7) / 8 * 8 * (((int64_t)m + 16 * tt - 1) / (16 * tt));
+}
+
+// Workgroups of 512 threads, in a grid of less than 2^32 threads
+bool grid_ok(int64_t n, int m, int rt) { return workgroups(n, m, rt) < (1 << 23); }
+
 template <typename K>
 hipError_t set_lds(K kern, size_t lds) {
     return lds > 65536 ? hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)
@@ -579,8 +590,7 @@ hipError_t launch_dense(const ProjGemmParams& p, hipStream_t st) {
     const auto kern = skinny_dense_kernel<RT, TT, S, NW>;
     const hipError_t e = set_lds(kern, lds);
     if (e != hipSuccess) return e;
-    const int tiles = (p.N + 16 * RT - 1) / (16 * RT), blocks = (p.M + 16 * TT - 1) / (16 * TT);
-    hipLaunchKernelGGL(kern, dim3((unsigned)((tiles + 7) / 8 * 8 * blocks)), dim3(64 * NW), lds, st, p, blocks);
+    hipLaunchKernelGGL(kern, dim3((unsigned)workgroups(p.N, p.M, RT)), dim3(64 * NW), lds, st, p, (p.M + 16 * TT - 1) / (16 * TT));
     return hipGetLastError();
 }
 
@@ -593,8 +603,7 @@ hipError_t launch_affine(const ProjGemmParams& p, const SkinnyRoute& route, hipS
     const hipError_t e = set_lds(kern, lds);
     if (e != hipSuccess) return e;
     const int tiles = (p.N + 16 * RT - 1) / (16 * RT), blocks = (p.M + 16 * TT - 1) / (16 * TT);
-    const unsigned grid = ROUTED ? (unsigned)(tiles * (route.experts + 1 + route.slots))
-                                 : (unsigned)((tiles + 7) / 8 * 8 * blocks);
+    const unsigned grid = (unsigned)(ROUTED ? tiles * (route.experts + 1 + route.slots) : workgroups(p.N, p.M, RT));
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * NW), lds, st, p, route, blocks);
     return hipGetLastError();
 }
@@ -620,7 +629,7 @@ bool affine_rows_ok(const ProjGemmParams& p) {
 bool skinny_gemm_ok(const ProjGemmParams& p) {
     if (p.M <= 0 || p.N <= 0 || p.K < 32 || p.K % 32 || ((uintptr_t)p.x & 15) || p.ldx % 8 || p.ldx < p.K) return false;
     if ((int64_t)64 * p.ldx * 2 >= (1 << 30)) return false;  // byte offsets of one token block's rows
-    if (((int64_t)p.N / 16 + 8) * ((int64_t)p.M / 16 + 1) > INT32_MAX) return false;  // workgroups
+    if (!grid_ok(p.N, p.M, p.packed ? 2 : 3)) return false;
     if (p.packed) return affine_rows_ok(p);
     return p.w && ((uintptr_t)p.w & 15) == 0 && p.ldw % 8 == 0 && p.ldw >= p.K && (int64_t)64 * p.ldw * 2 < (1 << 30);
 }
@@ -631,9 +640,6 @@ bool skinny_routed_ok(const ProjGemmParams& p, const SkinnyRoute& route) {
 }
 
 namespace {
-
-// Token tiles of 16 per workgroup
-int token_tiles(int m) { return m <= 16 ? 1 : (m <= 32 ? 2 : 4); }
 
 // Time of a dense launch with RT row tiles per workgroup, in units of one row
 // tile's weights per CU: workgroups run in rounds of one per CU, and a token
@@ -650,7 +656,7 @@ double dense_cost(int64_t n, int m, int rt, int cus) {
 int dense_rt(int64_t n, int m, int cus) {
     int best = 3;
     for (int rt = 2; rt >= 1; --rt)
-        if (dense_cost(n, m, rt, cus) < dense_cost(n, m, best, cus)) best = rt;
+        if (grid_ok(n, m, rt) && dense_cost(n, m, rt, cus) < dense_cost(n, m, best, cus)) best = rt;
     return best;
 }
 

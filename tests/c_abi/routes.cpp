@@ -38,4 +38,55 @@ int route_topk_sorts(int rows, int available, int ratio, int start_pos, int sele
     return mr::topk_sorts_whole(p, cus);
 }
 
+// mr::ProjRoute of bf16 tokens through a dense weight (group 0) or a 4-bit affine
+// one; tile_rows: token rows of a tile where the route has tiles
+int route_projection(int tokens, int out_features, int in_features, int group, int scale_dtype, int x_pad, int y_f32,
+                     int cus, int* tile_rows) {
+    mr::ProjGemmParams p{};
+    p.x = (const uint16_t*)at(1);
+    p.ldx = in_features + x_pad;
+    if (group) {
+        p.packed = at(2);
+        p.scales = at(3);
+        p.biases = at(4);
+        p.scale_dtype = scale_dtype;
+        p.group = group;
+        p.bits = 4;
+    } else {
+        p.w = (const uint16_t*)at(2);
+        p.ldw = in_features;
+    }
+    p.y = at(5);
+    p.ldy = out_features;
+    p.y_f32 = y_f32;
+    p.M = tokens;
+    p.N = out_features;
+    p.K = in_features;
+    const mr::ProjRoute r = mr::proj_route(p, cus);
+    const int64_t n_tiles = (out_features + 255) / 256;
+    *tile_rows = r == mr::PROJ_TILES         ? mr::proj_gemm_rows(n_tiles, tokens, cus)
+                 : r == mr::PROJ_GROUP_TILES ? mr::affine_gemm_rows(n_tiles, tokens, in_features, cus)
+                                             : 0;
+    return r;
+}
+
+// -1: a GEMV per pair
+int route_gather(int tokens, int experts, int per_token, int out_features, int in_features, int group) {
+    mr::ProjGemmParams p{};
+    p.x = (const uint16_t*)at(1);
+    p.ldx = in_features;
+    p.packed = at(2);
+    p.scales = at(3);
+    p.biases = at(4);
+    p.group = group;
+    p.bits = 4;
+    p.y = at(5);
+    p.ldy = out_features;
+    p.M = tokens;
+    p.N = out_features;
+    p.K = in_features;
+    const mr::SkinnyRoute r{(const int32_t*)at(6), tokens * per_token, per_token, experts, 0, 0};
+    return mr::skinny_routed_better(r.pairs, experts, p.N, p.K) && mr::skinny_routed_ok(p, r) ? mr::PROJ_FEW : -1;
+}
+
 }  // extern "C"

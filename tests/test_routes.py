@@ -52,3 +52,24 @@ def test_index_scores_kernel(routes, tokens, keys, many):
 def test_short_rows_sorted_or_selected(routes, rows, keys, ratio, start, few):
     for selected in sorted({1, few, few + 1, 2 * few + 1, min(512, keys), keys} - {0}):
         assert bool(routes.route_topk_sorts(rows, keys, ratio, start, selected, CUS)) == (selected > few), selected
+
+
+GEMV, FEW, TILES, GROUP_TILES = range(4)  # ProjRoute
+
+
+def projection(routes, tokens, out_f, in_f, group=0, sdt="bf16", x_pad=0, ydt="bf16"):
+    rows = C.c_int()
+    r = routes.route_projection(tokens, out_f, in_f, group, ("bf16", "f16", "f32").index(sdt), x_pad, int(ydt == "f32"),
+                                CUS, C.byref(rows))
+    return r, rows.value
+
+
+@pytest.mark.parametrize("tokens,out_f,in_f,route", [
+    (65536, 131073, 64, FEW),        # 5.6e6 workgroups of 512 threads
+    (131072, 262145, 64, GEMV),      # more threads than a grid has
+    (2 ** 31 - 1, 7, 64, GEMV),
+    (2 ** 31 - 1, 1001, 64, GEMV),
+    (131072, 262144, 64, TILES),     # rows that the 128-row tiles take
+])
+def test_few_token_tiles_fit_a_grid(routes, tokens, out_f, in_f, route):
+    assert projection(routes, tokens, out_f, in_f)[0] == route
