@@ -70,6 +70,12 @@ int route_projection(int tokens, int out_features, int in_features, int group, i
     return r;
 }
 
+// whether projections of `rows` weight rows in all, of the same tokens, run as one
+// stacked launch of large tiles (the others being takeable by both kinds)
+int route_stack(int tokens, int rows, int in_features, int affine, int cus) {
+    return tokens >= mr::PROJ_GEMM_MIN_TOKENS && !mr::skinny_gemm_better(rows, tokens, in_features, affine, cus);
+}
+
 // -1: a GEMV per pair
 int route_gather(int tokens, int experts, int per_token, int out_features, int in_features, int group) {
     mr::ProjGemmParams p{};

@@ -140,6 +140,18 @@ def test_affine_rotary_input_norm(M):
     check_prefill_block(M, d, C5, True, "prefill-block-affine-rotary")
 
 
+# 4-bit weights, fixed-width attention, a gate: q_a, kv_a (whose rows end inside a
+# tile) and g_proj in one launch of large tiles from about 600 tokens
+STACK = dict(hidden=2048, q_lora_rank=512, heads=16, nope=128, rope=64, v=128, kv_rank=512)
+
+
+@pytest.mark.parametrize("T,position", [(601, 30), (1270, 0)])
+def test_affine_stacked_projections(M, T, position):
+    print(f"prefill block affine, stacked projections T={T} position={position}", flush=True)
+    d = MI.prefill_block_inputs(T, position, f"pbst.{T}", affine=True, input_norm=True, **STACK)
+    check_prefill_block(M, d, STACK, False, f"prefill-block-affine-stack-{T}")
+
+
 def test_affine_any_width_rotary(M):
     dims = dict(hidden=256, q_lora_rank=64, heads=8, nope=24, rope=8, v=40, kv_rank=64)
     print("prefill block affine any-width rotary T=20 position=9", flush=True)

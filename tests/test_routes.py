@@ -1,6 +1,7 @@
 """The rules that choose a kernel for a call, on the CPU: tests/c_abi/routes.cpp
 calls them in the library with the sizes of a call and 256 compute units."""
 import ctypes as C
+import itertools
 import os
 import shutil
 import subprocess
@@ -8,6 +9,9 @@ import subprocess
 import pytest
 
 import minirun_hip as M
+import test_gpu_few_tokens as few_tokens
+import test_gpu_prefill_block as prefill_block
+import test_gpu_proj_gemm as proj_gemm
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CUS = 256
@@ -73,3 +77,97 @@ def projection(routes, tokens, out_f, in_f, group=0, sdt="bf16", x_pad=0, ydt="b
 ])
 def test_few_token_tiles_fit_a_grid(routes, tokens, out_f, in_f, route):
     assert projection(routes, tokens, out_f, in_f)[0] == route
+
+
+def parameters(test):
+    """The parameter sets of a test function, as dicts."""
+    axes = []
+    for mark in test.pytestmark:
+        if mark.name == "parametrize":
+            names = [n.strip() for n in mark.args[0].split(",")]
+            axes.append([dict(zip(names, v if len(names) > 1 else (v,))) for v in mark.args[1]])
+    return [{k: v for d in combo for k, v in d.items()} for combo in itertools.product(*axes)]
+
+
+@pytest.mark.parametrize("test,route", [
+    (proj_gemm.test_linear_tiles, TILES), (proj_gemm.test_affine_tiles, TILES),
+    (proj_gemm.test_linear_mfma_k3_shapes, TILES), (proj_gemm.test_affine_mfma_block_shapes, GROUP_TILES),
+    (proj_gemm.test_linear_mfma_edges, FEW),
+    (few_tokens.test_linear_few_tokens, FEW), (few_tokens.test_affine_few_tokens, FEW),
+    (few_tokens.test_affine_many_tokens, GROUP_TILES),
+])
+def test_gpu_tests_run_what_they_name(routes, test, route):
+    """Each size of a GPU test of one kernel goes to that kernel."""
+    for c in parameters(test):
+        affine = "affine" in test.__name__
+        got = projection(routes, c.get("tokens", proj_gemm.T_FULL), c["out_f"], c["in_f"],
+                         c.get("group", 64) if affine else 0, c.get("sdt", "bf16"), c.get("x_pad", 0), c.get("ydt", "f32"))
+        if test is few_tokens.test_linear_few_tokens and c["out_f"] > 12000 and c["tokens"] > 64:
+            assert got[0] == TILES  # the widest shape leaves the few-token tiles first
+            continue
+        assert got[0] == route, (c, got)
+        assert got[1] == c.get("rows", got[1]), (c, got)
+
+
+def test_gpu_tests_reach_both_tile_heights(routes):
+    heights = {projection(routes, c["tokens"], c["out_f"], c["in_f"], c["group"], c["sdt"], c["x_pad"], c["ydt"])[1]
+               for c in parameters(few_tokens.test_affine_many_tokens)}
+    assert heights == {64, 128}
+
+
+def test_gpu_affine_edges_run_both_kinds(routes):
+    for c in parameters(proj_gemm.test_affine_mfma_edges):
+        r = projection(routes, c["tokens"], c["out_f"], c["in_f"], c["group"], c["sdt"], c["x_pad"], c["ydt"])[0]
+        assert r == (FEW if c["group"] % 64 == 0 else TILES), c
+
+
+@pytest.mark.parametrize("test", [few_tokens.test_affine_non_finite, few_tokens.test_affine_non_finite_rows,
+                                  few_tokens.test_rows_do_not_see_what_follows_them])
+def test_gpu_tests_of_odd_values_run_both_kinds(routes, test):
+    for c in parameters(test):
+        if not c.get("experts"):
+            out_f = c.get("out_f", 6000 if c["tokens"] > 64 else 40)
+            r = projection(routes, c["tokens"], out_f, c["in_f"], 64, c.get("sdt", "bf16"), 64, "f32")[0]
+            assert r == (FEW if c["tokens"] < 100 else r) and r in (FEW, GROUP_TILES), c
+    assert {projection(routes, c["tokens"], c.get("out_f", 6000), c["in_f"], 64)[0]
+            for c in parameters(test) if c["tokens"] > 64 and not c.get("experts")} >= {GROUP_TILES}
+
+
+def test_gpu_cross_path_test_runs_three_paths(routes):
+    for group, large in ((64, GROUP_TILES), (0, TILES)):
+        got = [projection(routes, t, 1536, 7168, group, ydt="f32")[0] for t in proj_gemm.CROSS_TOKENS]
+        assert got == [GEMV, FEW, large]
+
+
+def gather(routes, c):
+    return routes.route_gather(c["tokens"], c["experts"], c["per_token"], c["out_f"], c["in_f"], c["group"])
+
+
+def test_gpu_gather_tests_run_what_they_name(routes):
+    assert all(gather(routes, c) == -1 for c in parameters(few_tokens.test_gather_few_pairs))
+    assert all(gather(routes, c) == FEW for c in parameters(few_tokens.test_gather_tokens_an_expert_together))
+    for c in parameters(few_tokens.test_rows_do_not_see_what_follows_them):
+        if c["experts"]:
+            assert gather(routes, dict(c, per_token=2, out_f=400, group=64)) == FEW, c
+
+
+@pytest.mark.parametrize("tokens,experts,per_token,out_f,in_f,together", [
+    (16, 128, 8, 768, 2048, False), (32, 128, 8, 768, 2048, True),   # two pairs an expert
+    (32, 64, 4, 512, 1024, False), (40, 64, 4, 512, 1024, True),     # enough work
+    (64, 1, 1, 768, 2048, False), (200, 1, 1, 768, 2048, True),
+    (200, 4000, 64, 768, 2048, False),                               # more experts than a workgroup counts
+])
+def test_gather_rule(routes, tokens, experts, per_token, out_f, in_f, together):
+    assert routes.route_gather(tokens, experts, per_token, out_f, in_f, 64) == (FEW if together else -1)
+
+
+def test_gpu_prefill_block_tests_run_stacked(routes):
+    """The 4-bit block test of many tokens takes its q_a, kv_a and g_proj as one
+    launch, in tiles of both heights."""
+    d, heights = prefill_block.STACK, set()
+    rows = d["q_lora_rank"] + d["kv_rank"] + d["rope"] + d["heads"] * d["v"]
+    for c in parameters(prefill_block.test_affine_stacked_projections):
+        assert routes.route_stack(c["T"], rows, d["hidden"], 1, CUS)
+        tiles = sum(-(-n // 256) for n in (d["q_lora_rank"], d["kv_rank"] + d["rope"], d["heads"] * d["v"]))
+        heights.add(projection(routes, c["T"], 256 * tiles, d["hidden"], 64)[1])
+    assert heights == {64, 128}
