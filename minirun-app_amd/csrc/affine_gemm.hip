@@ -12,13 +12,13 @@
 // too, four groups at a time (bf16 biases: one part, 3 of 16 k-slots a group;
 // else the six part products down to 2^-24).
 //
-// What bounds it: LDS and the DMA that fills it, then the matrix pipe.  7168 x
-// 16384, 1111 tokens: 361 us (724 before: two MFMAs per product, weights
-// dequantized by every workgroup between barriers); without its LDS reads of x
-// 285, without those and the DMA 207, without the scale multiply-adds 360.
-// Others, before -> now: 24576 x 1536, 1111 tokens 192 -> 161 us, 300 tokens 131
-// -> 51; 12288 x 7168, 1111 tokens 571 -> 311.  f32 outputs against 64 bits 1.1e-6
-// -> 2.6e-7 (K = 16384), 2.8e-7 -> 1.1e-7 (K = 1536).
+// What bounds it: LDS and the DMA that fills it, then the matrix pipe (busy 35% of
+// the cycles).  7168 x 16384, 1111 tokens: 356 us (698 before: two MFMAs per product,
+// weights dequantized by every workgroup between barriers); copies of the kernel
+// without its LDS reads of x took 285, without those and the DMA 207, without the
+// scale multiply-adds 360.  Others, before -> now: 24576 x 1536, 1111 tokens 192 ->
+// 161 us, 300 tokens 131 -> 51; 12288 x 7168, 1111 tokens 571 -> 311.  f32 outputs
+// against 64 bits 1.1e-6 -> 2.6e-7 (K = 16384), 2.8e-7 -> 1.1e-7 (K = 1536).
 //
 // A workgroup of 8 waves owns 32 MI tokens x 256 weight rows (MI = 4 or 2):
 // wave (h, c) takes rows 64 c .. + 63 of every second group (h), so each

@@ -378,7 +378,7 @@ mr_status mr_affine_matmul(const void* x, mr_dtype x_dtype, int32_t tokens, int6
     g.y_stride_token = y_stride;
     g.force_generic = !aligned16(w->packed);  // the fused kernel loads 16-byte row chunks
     if (tokens > 1 && x_dtype == MR_BF16) {
-        // MFMA: a few tokens in tiles of 16, or many in tiles of 128 and 256
+        // on MFMA, if a kernel takes it
         mr::ProjGemmParams q{};
         q.x = (const uint16_t*)x;
         q.ldx = x_stride;
@@ -423,7 +423,7 @@ mr_status mr_linear(const void* x, mr_dtype x_dtype, int32_t tokens, int64_t x_s
         return fail(MR_INVALID_SHAPE, "linear: an activation row of %lld %s values is under 16 bytes",
                     (long long)w->in_features, dtype_name(x_dtype));
     if (tokens > 1 && x_dtype == MR_BF16 && w->dtype == MR_BF16) {
-        // MFMA, as in mr_affine_matmul
+        // on MFMA, if a kernel takes it
         mr::ProjGemmParams q{};
         q.x = (const uint16_t*)x;
         q.ldx = x_stride;
@@ -1023,8 +1023,7 @@ mr_status mr_mla_decode_block(const mr_mla_block_args* a, void* stream) {
 // ---------------------------------------------------------------- prefill block
 namespace {
 
-// y[t] = W . x[t] for `tokens` bf16 rows into bf16 rows: MFMA tiles from
-// 64 tokens, the token-tiled GEMV below that
+// y[t] = W . x[t] for `tokens` bf16 rows into bf16 rows
 mr_status proj_rows(const void* x, int32_t tokens, int64_t x_stride, const mr_projection* w, void* y, int64_t y_stride,
                     void* stream) {
     return w->kind == MR_PROJ_AFFINE
@@ -1033,8 +1032,13 @@ mr_status proj_rows(const void* x, int32_t tokens, int64_t x_stride, const mr_pr
 }
 
 // Projections of the same bf16 rows into bf16 rows (n of them, up to 3):
-// one stacked MFMA launch when every weight takes the MFMA path and all are
-// dense bf16 or all affine, else one call each.
+// one stacked launch of large tiles when every weight takes them and all are
+// dense bf16 or all affine, else one call each.  Also one call each where few-token
+// tiles of all the rows together would be faster than the stack.  Whole blocks, us,
+// with few-token tiles throughout / large tiles throughout / by the rules: dense, 96
+// heads, 64 tokens 255 / 418 / 255, 160 tokens 360 / 404 / 317, 400 tokens 686 / 446
+// / 443; 4-bit, 128 heads, 64 tokens 227 / 462 / 227, 300 tokens 474 / 494 / 414;
+// the same with a gate, 96 heads, 200 tokens 446 / 417 / 365.
 mr_status proj_rows_stacked(const void* x, int32_t tokens, int64_t x_stride, const mr_projection* const* w,
                             void* const* y, const int64_t* y_stride, int n, void* stream) {
     mr::ProjGemmParams q[3];
@@ -1066,7 +1070,6 @@ mr_status proj_rows_stacked(const void* x, int32_t tokens, int64_t x_stride, con
         few = few && mr::skinny_gemm_ok(q[i]);
         rows += q[i].N;
     }
-    // a call each where the few-token tiles are faster than the stack's
     if (stack && !(few && mr::skinny_gemm_better(rows, tokens, q[0].K, w[0]->kind == MR_PROJ_AFFINE, mrc::cu_count()))) {
         const hipError_t e = mr::launch_proj_gemm_stack(q, n, mrc::cu_count(), (hipStream_t)stream);
         return e == hipSuccess ? MR_OK : hip_fail(e, "stacked projection launch");

@@ -234,6 +234,19 @@ __device__ __forceinline__ float wave_max(float v) {
 
 __device__ __forceinline__ float wave_sum(float v) { return group_sum(v, 64); }
 
+// Inclusive scan over the 64 lanes of a wave on DPP: row_shr 1, 2, 4, 8
+// inside rows of 16 lanes (lanes shifted in from outside the row add 0),
+// then row_bcast 15 / 31 carry each row's total into the rows above it.
+__device__ __forceinline__ uint32_t wave_scan_incl(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);
+    return v;
+}
+
 // v plus the value of lane l ^ 8 (DPP row_ror:8 rotates each 16-lane row by
 // 8, which is xor 8 there).
 __device__ __forceinline__ float xor8_sum(float v) {

@@ -225,13 +225,7 @@ __device__ __forceinline__ int sk_collect(const SkinnyRoute& route, int e, int l
             }
         const int valid = min(per, (left - first + 63) / 64);  // past it: zeros, or another wave's pairs
         hit &= valid <= 0 ? 0u : ~0u >> (32 - valid);
-        const int mine = __popc(hit);
-        int incl = mine;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int up = __shfl_up(incl, d);
-            if (l >= d) incl += up;
-        }
+        const int mine = __popc(hit), incl = (int)wave_scan_incl((uint32_t)mine);
         if (l == 63) sums[w] = incl;
         __syncthreads();
         int r = seen - lo + incl - mine;
@@ -286,12 +280,7 @@ __device__ __forceinline__ int2 sk_find_window(const SkinnyRoute& route, int o, 
     const int run = (n + NT - 1) / NT;
     int mine = 0;
     for (int j = tid * run; j < min(n, (tid + 1) * run); ++j) mine += max(0, bins[j] - 1) >> route.shift;
-    int incl = mine;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int up = __shfl_up(incl, d);
-        if (l >= d) incl += up;
-    }
+    int incl = (int)wave_scan_incl((uint32_t)mine);
     if (l == 63) sums[w] = incl;
     __syncthreads();
     for (int k = 0; k < w; ++k) incl += sums[k];
@@ -327,15 +316,16 @@ __device__ __forceinline__ int2 sk_find_window(const SkinnyRoute& route, int o, 
 // pairs and finds every route.slots-th of them, so that a hot expert is no chain
 // of passes.  They cost nothing that could be measured where no expert is hot.
 //
-// 2 waves and 16 tokens, eight workgroups a CU (at most 128 registers: 160 to 180
-// without the bound, and 8 to 40% slower): a workgroup is a chain of waits (ids,
-// rows, sums).  768 x 2048, 128 experts, 200 tokens of 8 slots, a GEMV per pair ->
-// now: spread 207 -> 45 us, half of the slots on one expert 192 -> 55, all on one
-// 191 -> 48 (318 and 609 when an expert was one workgroup per row tile).  2048 x
-// 768: 247 -> 45; 256 experts of 256 x 512, 2048 tokens 262 -> 45.  4 or 8 waves, 32
-// tokens, 64 or 128 rows each were slower with one workgroup per expert.
+// 2 waves and 16 tokens, six workgroups a CU (three waves a SIMD, at most 168
+// registers; at 128 and four waves 768 x 2048 takes 1 us more, 2048 x 768 5 less,
+// without a bound both are slower): a workgroup is a chain of waits (ids, rows,
+// sums).  768 x 2048, 128 experts, 200 tokens of 8 slots, a GEMV per pair -> now:
+// spread 207 -> 44 us, half of the slots on one expert 193 -> 54, all on one 190 ->
+// 45 (318 and 609 when an expert was one workgroup per row tile).  2048 x 768: 249
+// -> 48; 256 experts of 256 x 512, 2048 tokens 263 -> 50.  4 or 8 waves, 32 tokens,
+// 64 or 128 rows each were slower with one workgroup per expert.
 template <int RT, int TT, int S, int SDT, bool ROUTED, int NW>
-__global__ void __launch_bounds__(64 * NW, ROUTED ? 4 : 1) skinny_affine_kernel(ProjGemmParams p, SkinnyRoute route, int blocks) {
+__global__ void __launch_bounds__(64 * NW, ROUTED ? 3 : 1) skinny_affine_kernel(ProjGemmParams p, SkinnyRoute route, int blocks) {
     static_assert(RT <= 2, "one DMA of scales per entry");
     extern __shared__ __attribute__((aligned(16))) char lds[];
     constexpr int NI = RT + 4 * TT + 2, XOFF = 1024 * RT, SOFF = XOFF + 4096 * TT, ENTRY = SOFF + 512;
@@ -662,12 +652,17 @@ int dense_rt(int64_t n, int m, int cus) {
 
 }  // namespace
 
-// Against the 128-row tiles, both in rounds of one workgroup per CU.  Dense
-// (gemm.hip): a unit of dense_cost takes 1.65 ns per k (52 us at 12288 x 7168,
-// 64 tokens), a round of tiles 17.5 ns per k (128 us there).  Affine
-// (affine_gemm.hip): a round of 32 rows x 64 tokens takes 2.25 ns per k and 3.5
-// us (7168 x 16384: 128 tokens 81 us, there 194; 500 tokens 290, there 209;
-// 24576 x 1536: 64 tokens 24, there 25, 300 tokens 104, there 52).
+// Against the large tiles, both in rounds of one workgroup per CU.  Dense
+// (gemm.hip): a unit of dense_cost takes 1.65 ns per k (52 us at 12288 x 7168, 64
+// tokens), a round of tiles 17.5 ns per k (128 us there).  Over 14 shapes and 64 to
+// 512 tokens it never picks a kernel more than 5% slower than the tiles; the
+// few-token tiles would still be 5 to 25% faster at some sizes of 129 to 300 tokens
+// (12288 x 7168: 129 tokens 91 against 117 us, 192 tokens 105 against 121; 7168 x
+// 12288: 300 tokens 162 against 212).  Affine (affine_gemm.hip): a round of 32 rows
+// x 64 tokens takes 2.25 ns per k and 3.5 us (7168 x 16384: 128 tokens 81 us, there
+// 194; 500 tokens 290, there 209; 24576 x 1536: 64 tokens 24, there 25, 300 tokens
+// 104, there 52); over 13 shapes within 5% of the better one, but for 12288 x 7168
+// at 129 tokens (100 us, the other 94).
 bool skinny_gemm_better(int64_t n, int m, int k, bool affine, int cus) {
     if (m < PROJ_GEMM_MIN_TOKENS) return true;
     if (affine) {
@@ -698,17 +693,18 @@ hipError_t launch_skinny_gemm(const ProjGemmParams& p, int cu_count, hipStream_t
 // of waits, 6 to 13 us by K (8 experts of 1408 x 2048, 32 pairs, 92e6 weights:
 // 11.5 against 13.0 us, 40 pairs 17.8 against 13.1; 64 of 512 x 1024, 128 pairs,
 // 67e6: 10.4 against 10.6, with half of them to one expert 9.5 against 13.8, 160
-// pairs 18.2 against 10.7; 256 of 256 x 512, 512 pairs, 67e6: 13.1 against 11.6).
+// pairs 18.2 against 10.7; 256 of 256 x 512, 512 pairs, 67e6: 13.1 against 13.5,
+// with half to one 12.0 against 15.2, 768 pairs 17.7 against 14).
 bool skinny_routed_better(int64_t pairs, int64_t experts, int64_t n, int64_t k) {
-    return pairs >= 2 * experts && (double)pairs * (double)n * (double)k >= 40e6 + 30e3 * (double)k;
+    return pairs >= 2 * experts && (double)pairs * (double)n * (double)k >= std::max(68e6, 35e6 + 32.4e3 * (double)k);
 }
 
 // Windows of 16 pairs (one pass) up to twice the mean of an expert, so that few
 // experts have a second one; but where the experts alone do not fill the GPU, four
 // workgroups a CU, no more than lets the windows fill it (one expert of 768 x 2048,
-// 512 pairs: 17 us, 61 by the GEMV).  As many workgroups for the windows that
+// 512 pairs: 16.5 us, 61 by the GEMV).  As many workgroups for the windows that
 // follow a first one: half as many took 1.5 times as long at 2048 x 768, 200 tokens
-// of 8 slots all on one expert (67 us now, 248 by the GEMV).
+// of 8 slots all on one expert (62 us now, 248 by the GEMV).
 hipError_t launch_skinny_routed(const ProjGemmParams& p, const SkinnyRoute& r, int cu_count, hipStream_t st) {
     SkinnyRoute route = r;
     const int tiles = (p.N + 31) / 32;

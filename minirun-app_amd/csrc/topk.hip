@@ -51,19 +51,6 @@ __device__ __forceinline__ uint32_t ordered_bits(float f) {
 
 // Inclusive scan of one value per thread over the block; `sh` holds one
 // word per wave.  Every thread of the block must call it.
-// Inclusive scan over the 64 lanes of a wave on DPP: row_shr 1, 2, 4, 8
-// inside rows of 16 lanes (lanes shifted in from outside the row add 0),
-// then row_bcast 15 / 31 carry each row's total into the rows above it.
-__device__ __forceinline__ uint32_t wave_scan_incl(uint32_t v) {
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);
-    return v;
-}
-
 template <int NT>
 __device__ __forceinline__ uint32_t block_scan_incl(uint32_t v, uint32_t* sh) {
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
