@@ -247,12 +247,19 @@ mr_status mr_affine_dequantize(const mr_affine_weight *w, void *out, mr_dtype ou
  * transpose fixed (W is [out, in]).  x: [tokens, in] bf16 or f32 with row
  * stride x_stride; y: [tokens, out] bf16 or f32 with row stride y_stride;
  * fp32 accumulation.  4-bit / group-64 / bf16 x / one token runs the fused
- * dequant-GEMV; 64 or more bf16 tokens of a 4-bit weight whose group is a
- * multiple of 32 (in_features a multiple of 32, out_features of 8, 16-byte
- * aligned x and y rows) run on MFMA: each k-tile dequantized into LDS and
- * split into two bf16 operands (hi = bf16(w), lo = bf16(w - hi)), so each
- * product misses x * w by at most 2^-18 |w|; other shapes run a generic
- * kernel. */
+ * dequant-GEMV.  Two or more bf16 tokens of a 4-bit weight run on MFMA:
+ *   - groups of a multiple of 64 (16-byte aligned x rows and packed words, 4-byte
+ *     aligned scales and biases; 2-byte scales: an even number of them): the
+ *     group sums of x * q and of x, then scale and bias in fp32, so an
+ *     output's error is that of fp32 sums of terms |x| (|scale| q + |bias|), also
+ *     where scale * q + bias nearly cancels; outputs that are not finite that way
+ *     hold what the dequantized weights give;
+ *   - other groups of a multiple of 32, 64 or more tokens (in_features a multiple
+ *     of 32, out_features of 8, 16-byte aligned x and y rows): each k-tile
+ *     dequantized into LDS and split into two bf16 operands (hi = bf16(w), lo =
+ *     bf16(w - hi)), so each product misses x * w by at most 2^-18 |w|.
+ * Other shapes run a generic kernel.  The order of a token's sums, and so its
+ * last bits, depends on the kernel, which depends on the tokens of the call. */
 mr_status mr_affine_matmul(const void *x, mr_dtype x_dtype, int32_t tokens, int64_t x_stride,
                            const mr_affine_weight *w, void *y, mr_dtype y_dtype, int64_t y_stride,
                            void *stream);
@@ -278,8 +285,9 @@ mr_status mr_tile_upload(void *device_dst, const void *pinned_src, int64_t bytes
  * may repeat; y: [tokens][experts_per_token][out] bf16 or f32, dense.  The
  * reference's preconditions (a stacked weight, indices matching the token
  * count) return MR_INVALID_ARGUMENT with its message.  An expert id outside
- * [0, experts) yields a zero row (MLX leaves it undefined).  4-bit /
- * group-64 / bf16 x runs the fused dequant-GEMV per (token, slot). */
+ * [0, experts) yields a zero row (MLX leaves it undefined).  4-bit bf16 x
+ * runs the fused dequant-GEMV per (token, slot) (groups of 64), or, with many
+ * pairs and groups of a multiple of 64, each expert's pairs together on MFMA. */
 mr_status mr_affine_gather_matmul(const void *x, mr_dtype x_dtype, int32_t tokens, int64_t x_stride,
                                   const mr_affine_weight *w, int64_t experts, const int32_t *rhs_indices,
                                   int32_t experts_per_token, void *y, mr_dtype y_dtype, void *stream);
@@ -298,10 +306,10 @@ typedef struct mr_dense_weight {
 
 /* y[t, :] = x[t, :] . W^T for `tokens` rows of x (bf16 or f32, row stride
  * x_stride) into y (bf16 or f32, row stride y_stride), fp32 accumulation.
- * 64 or more bf16 tokens with a bf16 weight (in_features a multiple of 64,
- * out_features of 8, 16-byte aligned rows) run as an MFMA GEMM in tiles of
- * 256 (or 128) tokens x 256 outputs; otherwise every weight byte is read
- * once per tile of up to 8 tokens. */
+ * Two or more bf16 tokens with a bf16 weight (in_features a multiple of 32,
+ * 16-byte aligned rows) run on MFMA: a few in tiles of 16 tokens, many (from 64 on;
+ * out_features a multiple of 8) in tiles of 256 (or 128) tokens x 256 outputs;
+ * otherwise every weight byte is read once per tile of up to 8 tokens. */
 mr_status mr_linear(const void *x, mr_dtype x_dtype, int32_t tokens, int64_t x_stride, const mr_dense_weight *w,
                     void *y, mr_dtype y_dtype, int64_t y_stride, void *stream);
 
@@ -463,7 +471,7 @@ mr_status mr_mla_prefill(const mr_mla_prefill_args *args, void *stream);
  *          keys/values up-projected through kv_b (mr_mla_prefill)  (:159-206)
  *   out = o_proj(attn * sigmoid(g_proj(h)))  (gate when g_proj is given,
  *                                             :207-211)
- * Projections run over all T tokens (MFMA tiles from 64 tokens).  kv_b is
+ * Projections run over all T tokens, on MFMA from 2 tokens.  kv_b is
  * dense bf16 (K3's) or affine, dequantized to bf16 in the workspace.  Widths
  * as mr_mla_prefill takes them; qk_rope_dim even.  rope_cos / rope_sin:
  * device [T][qk_rope_dim/2], the angles at positions position .. position+T-1

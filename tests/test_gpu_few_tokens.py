@@ -301,7 +301,7 @@ def routing(kind, tokens, experts, per_token):
 @pytest.mark.parametrize("tokens,experts,per_token,out_f,in_f,group,sdt,ydt", [
     (700, 16, 6, 98, 192, 64, "bf16", "bf16"),   # 4200 pairs: two scans; an odd group count, ragged rows
     (300, 128, 8, 40, 1152, 128, "f32", "f32"),
-    (700, 3, 6, 70, 192, 64, "f16", "f32"),
+    (700, 3, 6, 90, 192, 64, "f16", "f32"),
     (6000, 4, 2, 96, 64, 64, "bf16", "f32"),     # more windows of one expert than workgroups for them
 ])
 def test_gather_tokens_an_expert_together(M, tokens, experts, per_token, out_f, in_f, group, sdt, ydt, kind):
